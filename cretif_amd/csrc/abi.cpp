@@ -522,6 +522,9 @@ PrefillWs prefill_ws(int M, int H, int Hkv, int D, int kv_len) {
     w.vh = w.kt + Hkv * T4 * D;
     w.sc = w.vh + Hkv * T4 * D;
     w.total = 16 + 4 * (w.sc + H * rows * T4);
+    // head_dim 64 and 128 take the prompt attention kernel from 32 rows, whose workspace is usually the smaller
+    if (cri::detail::prompt_attention_supported(M, D) && H % Hkv == 0)
+        w.total = std::max(w.total, cri::detail::prompt_attention_workspace_bytes(M, H, Hkv, D, kv_len));
     return w;
 }
 }  // namespace
@@ -556,6 +559,13 @@ int cri_prefill_attention(const float* Q, int ldq, const float* K_cache, const f
         return fail(CRI_ERR_SHAPE, fn, "workspace of " + std::to_string(workspace_bytes) + " bytes, " +
                                            std::to_string(w.total) + " needed");
     clear_pending_error();
+    if (cri::detail::prompt_attention_supported(M, head_dim)) {
+        const int rc = cri::detail::launch_prompt_attention(Q, ldq, K_cache, V_cache, output, n_heads * head_dim, M,
+                                                            n_heads, n_kv_heads, head_dim, nullptr, pos + 1,
+                                                            static_cast<int>(kv_len), scale, workspace, s);
+        if (rc == cri::detail::kFailed) return fail(CRI_ERR_LAUNCH, fn, "launch failed");
+        if (rc == 0) return check_launch(fn);
+    }
     int* pos_dev = static_cast<int*>(workspace);
     float* base = reinterpret_cast<float*>(static_cast<char*>(workspace) + 16);
     if (cri::detail::launch_pos_set(pos_dev, pos, s) != 0) return fail(CRI_ERR_LAUNCH, fn, "launch failed");

@@ -738,8 +738,8 @@ __global__ __launch_bounds__(256) void decode_attn_combine64_kernel(const float*
 namespace detail {
 
 // merge the chunk records of every (row, head)
-static void launch_combine(const float* ws, float* out, int n_heads, int rows, int D, int nchunks, long ldo,
-                           hipStream_t stream) {
+void launch_attention_combine(const float* ws, float* out, int n_heads, int rows, int D, int nchunks, long ldo,
+                              hipStream_t stream) {
     const dim3 grid(n_heads, static_cast<unsigned>(rows));
     if (D == 64 && nchunks <= dev::kCombine64MaxChunks)
         hipLaunchKernelGGL(dev::decode_attn_combine64_kernel, grid, dim3(256), 0, stream, ws, out, nchunks, ldo);
@@ -825,7 +825,7 @@ int launch_decode_attention_rows(const float* Q, long ldq, const float* K, const
             hipLaunchKernelGGL(dev::decode_attn_mrow_kernel<false>, dim3(static_cast<unsigned>(wgs)),
                                dim3(64 * dev::kMrWaves), 0, stream, Q, K, V, ws, G, n_kv_heads, rows, kv_dev, kv0,
                                qscale, nchunks, ldq, nullptr, ldo);
-        if (!direct) launch_combine(ws, out, n_heads, rows, D, nchunks, ldo, stream);
+        if (!direct) launch_attention_combine(ws, out, n_heads, rows, D, nchunks, ldo, stream);
         return 0;
     }
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(rows));
@@ -835,7 +835,7 @@ int launch_decode_attention_rows(const float* Q, long ldq, const float* K, const
     else
         hipLaunchKernelGGL((dev::decode_attn_split_kernel<kSplitHeadsPerWave, 8>), grid, dim3(256 / kSplitHeadsPerWave),
                            0, stream, Q, K, V, ws, G, n_kv_heads * D, D, kv_dev, kv0, qscale, nchunks, nhq, ldq);
-    launch_combine(ws, out, n_heads, rows, D, nchunks, ldo, stream);
+    launch_attention_combine(ws, out, n_heads, rows, D, nchunks, ldo, stream);
     return 0;
 }
 

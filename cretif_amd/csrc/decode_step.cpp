@@ -28,8 +28,8 @@ namespace {
 
 // Batches up to this many tokens take the fused RMSNorm / SwiGLU prologues.
 constexpr int kFusedMaxBatch = 16;
-// Larger batches (a prompt) run attention on the multi-row split kernel at head_dim 64, otherwise
-// through batched_matmul_gqa in row blocks of cri::detail::kPromptRows rows (the scores workspace
+// Larger batches (a prompt) run attention on the prompt kernel (from kPromptAttnMinRows rows at
+// head_dim 64 and 128), below that at head_dim 64 on the multi-row split kernel, otherwise through batched_matmul_gqa in row blocks of cri::detail::kPromptRows rows (the scores workspace
 // holds n_heads x that x max_seq_len floats).
 using cri::detail::kPromptRows;
 
@@ -177,10 +177,12 @@ DecodeStep::DecodeStep(const DecodeStepConfig& c) : cfg_(c) {
     act_ = Tensor::empty({MB, static_cast<int64_t>(c.intermediate_size)});
     ffn_out_ = Tensor::empty({MB, static_cast<int64_t>(c.dim)});
     // records for the larger of the one-row and the multi-row chunk counts (the split attention
-    // serves batches of up to kFusedMaxBatch rows, and prompts too where the multi-row kernel
-    // takes them: head_dim 64)
-    prompt_mrow_ = MB > kFusedMaxBatch && cri::detail::decode_attention_rows_mrow(static_cast<int>(MB), c.head_dim);
-    const int64_t arows = prompt_mrow_ ? MB : std::min<int64_t>(MB, kFusedMaxBatch);
+    // serves batches of up to kFusedMaxBatch rows, and the shortest prompts where the multi-row
+    // kernel takes them)
+    const bool fused = cri::detail::prompt_attention_supported(cri::detail::kPromptAttnMinRows, c.head_dim);
+    const int64_t short_rows = std::min<int64_t>(MB, fused ? cri::detail::kPromptAttnMinRows - 1 : cri::detail::kPromptRows);
+    prompt_mrow_ = fused && cri::detail::decode_attention_rows_mrow(kFusedMaxBatch + 1, c.head_dim);
+    const int64_t arows = prompt_mrow_ ? short_rows : std::min<int64_t>(MB, kFusedMaxBatch);
     // the most records any batch size up to arows writes (its rows x heads x chunks; the chunk count
     // falls as the rows grow)
     int64_t recs = 0;
@@ -203,8 +205,13 @@ DecodeStep::DecodeStep(const DecodeStepConfig& c) : cfg_(c) {
     argmax_count_ = Tensor::zeros({MB});
     res_parts_ = Tensor::empty({static_cast<int64_t>(cri::kResMaxSplits) * c.dim});
     norm_ss_ = Tensor::zeros({256});
+    if (fused && MB >= cri::detail::kPromptAttnMinRows) {
+        const long bytes = cri::detail::prompt_attention_workspace_bytes(c.max_batch, c.n_heads, c.n_kv_heads, c.head_dim,
+                                                                         c.max_seq_len);
+        prompt_ws_ = Tensor::empty({(bytes + 3) / 4});
+    }
     if (MB > kFusedMaxBatch && !prompt_mrow_) {
-        const int64_t rows = std::min<int64_t>(MB, kPromptRows), T4 = round4(c.max_seq_len);
+        const int64_t rows = short_rows, T4 = round4(c.max_seq_len);
         gqa_q_ = Tensor::empty({c.n_heads * rows * c.head_dim});
         gqa_o_ = Tensor::empty({c.n_heads * rows * c.head_dim});
         gqa_k_ = Tensor::empty({c.n_kv_heads * T4 * c.head_dim});
@@ -496,7 +503,14 @@ void DecodeStep::attn_block(Layer& L, int li, int M, int& cur, const float*& res
                      "rope/append");
     // row m attends to positions [0, pos + m] (ref:src/attention.cu:60-75; one token: :410-511)
     const float scale = 1.0f / std::sqrt(static_cast<float>(cfg_.head_dim));
-    if (M > kFusedMaxBatch && !prompt_mrow_) {
+    if (M > kFusedMaxBatch && cri::detail::prompt_attention_supported(M, cfg_.head_dim)) {
+        // the plan depends on the cache's size, not on the position, so a graph computes what the
+        // eager step does
+        check_status(cri::detail::launch_prompt_attention(q, ldq, k_cache(li), v_cache(li), ctx_.data_as<float>(), QD, M,
+                                                          cfg_.n_heads, cfg_.n_kv_heads, cfg_.head_dim, pos, 1,
+                                                          cfg_.max_seq_len, scale, prompt_ws_.data(), s),
+                     "prompt attention");
+    } else if (M > kFusedMaxBatch && !prompt_mrow_) {
         // a prompt: Q K^T and P V through batched_matmul_gqa around a causal softmax, in row blocks
         // (ref:src/attention.cu:809-871); the products span the cache positions the block can see,
         // rounded up to a multiple of 4 -- the whole cache when recording a graph, which is then

@@ -250,6 +250,23 @@ bool decode_attention_rows_mrow(int rows, int head_dim);
 int launch_decode_attention_rows(const float* Q, long ldq, const float* K, const float* V, float* out, long ldo,
                                  int rows, int n_heads, int n_kv_heads, int head_dim, const int* kv_dev, int kv0,
                                  int nchunks, float scale, float* ws, hipStream_t stream);
+// merges the records [rows][n_heads][nchunks][head_dim + 4] of (max, sum, 2 pad, acc) into out
+void launch_attention_combine(const float* ws, float* out, int n_heads, int rows, int D, int nchunks, long ldo,
+                              hipStream_t stream);
+
+// causal attention of a prompt's M query rows (prompt_attention.hip; head_dim 64 and 128): row m at
+// Q + m ldq sees the first kv0 + m positions (+ *kv_dev when kv_dev is not null), at most kv_max in
+// all; output row m at out + m ldo (16-byte aligned, ldo % 4 == 0); ws: 16-byte aligned,
+// prompt_attention_workspace_bytes of it, written before it is read.  From 32 rows: there the products
+// it replaces ran on v_mfma_f32_32x32x2 and were further from float64 (1.5e-7 against 1.2e-7 at 32
+// rows, 8.6e-7 against 2.2e-7 at position 2000); below, on fp32 FMAs, they were closer (8.6e-8
+// against 1.0e-7 at 17 rows) and stay
+constexpr int kPromptAttnMinRows = 32;
+bool prompt_attention_supported(int M, int head_dim);
+long prompt_attention_workspace_bytes(int M, int n_heads, int n_kv_heads, int head_dim, int kv_max);
+int launch_prompt_attention(const float* Q, long ldq, const float* K, const float* V, float* out, long ldo, int M,
+                            int n_heads, int n_kv_heads, int head_dim, const int* kv_dev, int kv0, int kv_max,
+                            float scale, void* ws, hipStream_t stream);
 
 // cri_fused_decode_attention_noalloc: its records live in a file-scope device array of this
 // many bytes (attention.hip); noalloc_scratch gives the current device's address of it

@@ -160,13 +160,14 @@ private:
     Tensor k_cache_, v_cache_, pos_dev_;
     Tensor hid_[2], normed_, qkv_, ctx_, attn_out_, ff_, act_, ffn_out_, attn_ws_, split_ws_, defer_ws_;
     Tensor argmax_part_, argmax_count_, rope_;
-    // batches above 16 rows (a prompt): attention through batched_matmul_gqa in row blocks of up to
-    // kPromptRows, on Q / K^T / V / scores / output workspaces (allocated when max_batch > 16)
+    // batches above 16 rows (a prompt): the prompt attention kernel on prompt_ws_ (head_dim 64 and
+    // 128, from 32 rows), the multi-row split attention (the rows below at head_dim 64), otherwise
+    // batched_matmul_gqa in row blocks of up to kPromptRows around a causal softmax, on Q / K^T / V /
+    // scores / output workspaces (allocated when max_batch > 16)
+    bool prompt_mrow_ = false;
+    Tensor prompt_ws_;
     Tensor gqa_q_, gqa_k_, gqa_v_, gqa_s_, gqa_o_;
     bool capturing_ = false;  // enqueue() is recording a graph: shapes independent of the position
-    // prompts (above 16 tokens) through the multi-row split attention (head_dim 64) instead of
-    // batched_matmul_gqa around a materialized causal softmax
-    bool prompt_mrow_ = false;
     Tensor res_parts_;    // the down projection's K-split partial sums at one token
     int res_splits_ = 0;  // > 0: the pending residual is that many partial sums in res_parts_
     // 2..16 tokens: the pending residual as the unreduced partial sums of the o projection, and

@@ -1,0 +1,103 @@
+"""The prompt attention kernel (cri_prefill_attention at head_dim 64 and 128 from 32 rows) at the
+edges of its tiles, query groups and chunks, against the oracle's decode attention row by row.
+
+Bar: 1e-5 normwise, the bar of every fp32 path.  The kernel's own error is the fp16 parts' (2^-24 of
+each operand and of each dropped product, about 4e-7 of a score of magnitude 8) plus fp32 sums over
+the positions, a few 1e-7 in all.
+"""
+import numpy as np
+import pytest
+import torch
+
+import cretif_amd as cri
+from conftest import normwise_rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def run(q, ldq, kc, vc, M, H, Hkv, D, pos, scale):
+    out = torch.full((M, H * D), float("nan"), device="cuda")
+    cri.prefill_attention(torch.from_numpy(q).cuda(), ldq, torch.from_numpy(kc).cuda(), torch.from_numpy(vc).cuda(),
+                          out, M, H, Hkv, D, pos, scale)
+    return out.cpu().numpy()
+
+
+def inputs(M, H, Hkv, D, pos, past=9):
+    rng = np.random.default_rng(1000 * M + pos + D + H)
+    ldq = (H + 2 * Hkv) * D
+    q = rng.standard_normal((M, ldq)).astype(np.float32)
+    kc = rng.standard_normal((pos + M + past, Hkv, D)).astype(np.float32)
+    vc = rng.standard_normal((pos + M + past, Hkv, D)).astype(np.float32)
+    kc[pos + M:] = np.nan  # rows past the prompt are never read into the products
+    vc[pos + M:] = np.nan
+    return q, ldq, kc, vc
+
+
+def rows_of(M):
+    return sorted({0, 1, M // 3, M // 2, M - 2, M - 1, *(r for r in (31, 32, 63, 64, 127, 128) if r < M)})
+
+
+# one query group and its remainder, groups that straddle rows (G = 3, 7), one head per KV head, tile
+# remainders, every chunk count from 16 down to one, two- and four-block workgroups, paired ones with an
+# even and an odd group count
+@pytest.mark.parametrize("H,Hkv,D,M,pos", [
+    (1, 1, 64, 32, 0), (7, 1, 64, 33, 31), (3, 1, 128, 37, 3), (8, 8, 128, 65, 0), (32, 8, 64, 64, 959),
+    (4, 1, 128, 300, 700), (32, 8, 64, 513, 0), (8, 8, 64, 1000, 24), (32, 8, 64, 1025, 0), (32, 8, 64, 2050, 0),
+    (32, 8, 128, 1030, 5), (32, 8, 128, 2049, 0),
+])
+def test_matches_oracle(orc, H, Hkv, D, M, pos):
+    q, ldq, kc, vc = inputs(M, H, Hkv, D, pos)
+    scale = np.float32(1.0 / np.sqrt(D))
+    got = run(q, ldq, kc, vc, M, H, Hkv, D, pos, scale)
+    assert np.isfinite(got).all()
+    for m in rows_of(M):
+        ref = orc.decode_attention(q[m, :H * D], kc, vc, H, Hkv, D, pos + m + 1, scale)
+        assert normwise_rel_err(got[m], ref) <= 1e-5, m
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("what", ["wide", "spread", "tiny_k", "big_q", "zero_v", "peak"])
+def test_ranges(orc, D, what):
+    """Operands of any finite magnitude: tile scales of their own, and the fp32 path where parts
+    would not be exact (V tiles 2^100 apart, a tile or a query below 2^-100, values of 2^127)."""
+    H, Hkv, M, pos = 4, 2, 70, 90
+    q, ldq, kc, vc = inputs(M, H, Hkv, D, pos)
+    if what == "wide":  # V tiles 2^40 apart, K tiles 2^20 apart (scores stay moderate)
+        vc[32:64] *= np.float32(2.0 ** -40)
+        kc[96:128] *= np.float32(2.0 ** -20)
+    elif what == "spread":
+        vc[:32] *= np.float32(2.0 ** -60)
+        vc[64:96] *= np.float32(2.0 ** 60)
+    elif what == "tiny_k":
+        kc *= np.float32(2.0 ** -104)
+        q *= np.float32(2.0 ** 100)
+    elif what == "big_q":
+        q[:] = np.float32(2.0 ** 126) * np.sign(q)
+        kc *= np.float32(2.0 ** -125)
+    elif what == "zero_v":
+        vc[:64] = 0
+    else:  # one score far above the rest, then a later higher one: the running maximum is raised late
+        kc[40] = 30 * q[0, :D]
+        kc[120] = 60 * q[0, :D]
+    scale = np.float32(1.0 / np.sqrt(D))
+    got = run(q, ldq, kc, vc, M, H, Hkv, D, pos, scale)
+    for m in rows_of(M):
+        ref = orc.decode_attention(q[m, :H * D], kc, vc, H, Hkv, D, pos + m + 1, scale)
+        assert normwise_rel_err(got[m], ref) <= 1e-5, m
+
+
+def test_nonfinite_keys_and_values():
+    """A NaN key or an infinite value reaches exactly the rows and heads that see it."""
+    H, Hkv, D, M = 4, 2, 64, 100
+    q, ldq, kc, vc = inputs(M, H, Hkv, D, 0)
+    clean = run(q, ldq, kc, vc, M, H, Hkv, D, 0, 0.125)
+    kc[50, 0, 3] = np.nan
+    vc[70, 1, 5] = np.inf
+    got = run(q, ldq, kc, vc, M, H, Hkv, D, 0, 0.125).reshape(M, H, D)
+    clean = clean.reshape(M, H, D)
+    assert np.isnan(got[50:, :2]).all()
+    assert normwise_rel_err(got[:50, :2], clean[:50, :2]) <= 1e-5
+    assert normwise_rel_err(got[:70, 2:], clean[:70, 2:]) <= 1e-5
+    assert np.isposinf(got[70:, 2:, 5]).all()
+    keep = [d for d in range(D) if d != 5]
+    assert normwise_rel_err(got[70:, 2:][..., keep], clean[70:, 2:][..., keep]) <= 1e-5
