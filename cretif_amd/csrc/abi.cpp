@@ -172,7 +172,7 @@ long long cri_matmul_workspace_bytes(int format, int M, int N, int K) {
     // above 16 rows: the prefill kernel's K split (formats and K it takes; the other kernels split nothing
     // a workspace would hold)
     if (M > kPrefillMinM)
-        return K % 256 == 0 ? static_cast<long long>(cri::detail::prefill_workspace_floats(M, N, K)) * 4 : 0;
+        return K % 256 == 0 ? static_cast<long long>(cri::detail::prefill_workspace_floats(format, M, N, K, false)) * 4 : 0;
     return static_cast<long long>(cri::detail::skinny_workspace_floats(M, N)) * 4;
 }
 
@@ -205,16 +205,22 @@ int cri_matmul_ws(int format, const float* A, const void* B, float* C, int M, in
         // the prefill GEMM's K split (few output tiles, e.g. 512 x 2048 x 8192): its partial sums go
         // to the workspace and a second launch adds them in split order, in place of atomics into a
         // zero-filled C (the same bits on every call)
-        const long long need = cri_matmul_workspace_bytes(format, M, N, K);
-        if (need > 0 && cri::detail::prefill_supported(format, M, N, K, A, B)) {
-            if (!workspace || workspace_bytes < need)
+        // (the 128-row tiles of a longer prompt split K too where the workspace holds the partial sums;
+        // a smaller one is enough for the 64-row tiles)
+        const long long need =
+            K % 256 == 0 ? static_cast<long long>(cri::detail::prefill_workspace_floats(format, M, N, K, true)) * 4 : 0;
+        if (cri::detail::prefill_supported(format, M, N, K, A, B)) {
+            if (need > 0 && (!workspace || workspace_bytes < need))
                 return fail(CRI_ERR_INVALID_ARGUMENT, fn,
                             "workspace of at least " + std::to_string(need) +
                                 " bytes needed (cri_matmul_workspace_bytes)");
-            if (!aligned(workspace, 16) || !aligned(C, 16) || N % 4 != 0)
+            const bool fits = aligned(workspace, 16) && aligned(C, 16) && N % 4 == 0;
+            if (need > 0 && !fits)
                 return fail(CRI_ERR_ALIGNMENT, fn, "workspace and C must be 16-byte aligned and N a multiple of 4");
-            ws = static_cast<float*>(workspace);
-            ws_floats = static_cast<long>(workspace_bytes / 4);
+            if (workspace && fits) {
+                ws = static_cast<float*>(workspace);
+                ws_floats = static_cast<long>(workspace_bytes / 4);
+            }
         }
     }
     // the format ids of cri.h are the library's internal ones

@@ -174,14 +174,16 @@ bool prefill_supported(int fmt, int M, int N, int K, const void* A, const void* 
 int launch_prefill(int fmt, const float* A, const void* B, float* C, int M, int N, int K, hipStream_t stream,
                    float* ws = nullptr, long ws_floats = 0, SplitSums* defer = nullptr, int defer_S = 0);
 // K splits of the prefill GEMM are chosen so that tiles x splits < 512; so at most this many
-// partial-sum floats (512 tiles of 64 x 256); splits past 16 take the atomics
-constexpr long kPrefillSplitFloats = 512L * 64 * 256;
+// partial-sum floats (512 tiles of 128 x 256); splits past 16 take the atomics
+constexpr long kPrefillSplitFloats = 512L * 128 * 256;
 // C[M, F] = SiLU(A gate^T) * (A up^T) for a stacked gate/up matrix B of 2F rows (gate first), the
 // product and the elementwise step in one launch (the SiLU * up of the separate kernel, bit for
 // bit); kDeclined where the tiles would need a K split (short prompts) or the kernel does not apply
 int launch_prefill_swiglu(int fmt, const float* A, const void* B, float* C, int M, int F, int K, hipStream_t stream);
-// floats of partial sums launch_prefill stores in a workspace for this shape (0: no K split)
-long prefill_workspace_floats(int M, int N, int K);
+// floats of partial sums launch_prefill stores in a workspace for this shape (0: no K split); least:
+// those of the 64-row kernel, without which the split it makes on its own would take atomics (the
+// 128-row kernel's split is only made where a workspace holds it)
+long prefill_workspace_floats(int fmt, int M, int N, int K, bool least);
 // C = the S partial sums of p added in split order (times p's RMSNorm row factor); M N % 4 == 0,
 // C and p.part 16-byte aligned, p.stride % 4 == 0 (mfma_skinny.hip)
 int launch_split_reduce(const SplitSums& p, float* C, int M, hipStream_t stream);

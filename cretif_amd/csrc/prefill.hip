@@ -38,6 +38,8 @@
 //     when the tiles cannot fill 256 CUs the k range is split over workgroups
 //     that add into a zeroed C with fp32 atomics, or, given a workspace, store
 //     their partial sums there for a fixed-order reduction;
+//   * where 128-row tiles fill the GPU too (prefill_plan), a second kernel takes
+//     them: each decoded weight feeds four MFMAs instead of two;
 //   * a stacked gate/up matrix can take a SiLU(gate) * up epilogue: a tile's
 //     128 output columns are 128 gate rows and the matching 128 up rows.
 // Activations outside fp16's comfortable range would lose the 1e-3 bound (a
@@ -47,6 +49,7 @@
 // the reference's per-element decode at the end of the tile (the fp16 MFMA
 // results of those rows are not stored).  Dequantized weights must fit fp16
 // (|x| < 65504), as every GGUF model's do.
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -569,6 +572,48 @@ struct PQ6K {
 template <int J>
 using pos_t = std::integral_constant<int, J>;
 
+// fp32 path for the flagged rows of a 64-row block starting at row m0 (bit ml: row m0 + ml): the
+// reference's per-element decode and a sequential fp32 sum over the workgroup's k range.  Thread ->
+// column nt * 256 + (tid & 255) of the rows of parity tid >> 8; swiglu: output column nt * 128 +
+// (tid & 127) of the rows of class tid >> 7 (mod 4), the gate and up sums over the whole k range (no
+// split), then SiLU(gate) * up.
+template <class W>
+__device__ __forceinline__ void flagged_rows(unsigned long long flagged, const float* __restrict__ A,
+                                             const uint8_t* __restrict__ B, float* __restrict__ out, int m0, int M, int N,
+                                             int K, long row_bytes, int nt, int s_begin, int s_end, bool add, int swiglu) {
+    const int fmt = W::kFmt, tid = threadIdx.x, F = N >> 1;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (swiglu) {
+        for (unsigned long long rest = flagged & (0x1111111111111111ull << (wave >> 1)); rest != 0; rest &= rest - 1) {
+            const int m = m0 + __builtin_ctzll(rest), col = nt * (kPTN / 2) + (tid & (kPTN / 2 - 1));
+            if (m >= M || col >= F) continue;
+            const float* x = A + static_cast<long>(m) * K;
+            const uint8_t* gp = B + static_cast<long>(col) * row_bytes;
+            const uint8_t* up = B + static_cast<long>(F + col) * row_bytes;
+            float g = 0.0f, v = 0.0f;
+            for (int k = 0; k < K; ++k) {
+                g = __builtin_fmaf(x[k], decode_row_elem(fmt, gp, k), g);
+                v = __builtin_fmaf(x[k], decode_row_elem(fmt, up, k), v);
+            }
+            out[static_cast<long>(m) * F + col] = silu_f(g) * v;
+        }
+        return;
+    }
+    for (unsigned long long rest = flagged & (0x5555555555555555ull << (wave >> 2)); rest != 0; rest &= rest - 1) {
+        const int m = m0 + __builtin_ctzll(rest), nn = nt * kPTN + (tid & 255);
+        if (m >= M || nn >= N) continue;
+        const float* x = A + static_cast<long>(m) * K;
+        const uint8_t* wp = B + static_cast<long>(nn) * row_bytes;
+        float sum = 0.0f;
+        for (int k = s_begin * kPKS; k < s_end * kPKS; ++k) sum = __builtin_fmaf(x[k], decode_row_elem(fmt, wp, k), sum);
+        float* cp = out + static_cast<long>(m) * N + nn;
+        if (add)
+            atomicAdd(cp, sum);
+        else
+            *cp = sum;
+    }
+}
+
 // dynamic LDS: two activation buffers of four step tiles, then one weight area per wave
 template <class W>
 constexpr int prefill_lds_bytes() {
@@ -910,8 +955,11 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
         if (ap == 0) rowflag[ar0 + 32 * i] = (v >= kPRowMax || (v > 0.0f && v < kPRowMin)) ? 1 : 0;
     }
     __syncthreads();
-    // the 64 flags as one wave-uniform mask (bit ml: row m0 + ml takes the fp32 path)
+    // the 64 flags as one wave-uniform mask (bit ml: row m0 + ml takes the fp32 path), tested in halves:
+    // with 256 registers the compiler put the amount of a 64-bit shift in v255, and this GPU then
+    // shifts by the first register of another wave
     const unsigned long long flagged = __ballot(rowflag[lane] != 0);
+    const uint32_t fl[2] = {static_cast<uint32_t>(flagged), static_cast<uint32_t>(flagged >> 32)};
 
     // lane: column n0 + fr, rows m0 + 32 u + 8 g + 4 h + r (accumulator 4 g + r); the stores
     // stream past the caches (the output is not read again by this kernel)
@@ -932,7 +980,7 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
         __syncthreads();
         const int j = tid & (kPTN / 2 - 1), col = nt * (kPTN / 2) + j;
         for (int ml = tid / (kPTN / 2); ml < kPTM; ml += kPThreads / (kPTN / 2))
-            if (ml < mrows && col < F && !((flagged >> ml) & 1ull))
+            if (ml < mrows && col < F && !(((ml < 32 ? fl[0] : fl[1]) >> (ml & 31)) & 1u))
                 __builtin_nontemporal_store(silu_f(ct[ml * kPTN + j]) * ct[ml * kPTN + kPTN / 2 + j],
                                             C + static_cast<long>(m0 + ml) * F + col);
     } else {
@@ -941,7 +989,7 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const int ml = 32 * u + 8 * (i >> 2) + 4 * h + (i & 3);
-                if (ml < mrows && n < N && !((flagged >> ml) & 1ull)) {
+                if (ml < mrows && n < N && !((fl[u] >> (ml & 31)) & 1u)) {
                     float* cp = out + static_cast<long>(m0 + ml) * N + n;
                     if (add)
                         atomicAdd(cp, acc[u][i]);
@@ -951,43 +999,324 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
             }
     }
 
-    // fp32 path for flagged rows: thread -> column nt * 256 + (tid & 255) of the flagged rows
-    // of parity tid >> 8, the reference's per-element decode and a sequential fp32 sum over
-    // this workgroup's k range
-    const int fmt = W::kFmt;
-    if (swiglu) {
-        // thread -> output column nt * 128 + (tid & 127) of the flagged rows of class tid >> 7 (mod
-        // 4): the gate and up sums over the whole k range (no split), then SiLU(gate) * up
-        for (unsigned long long rest = flagged & (0x1111111111111111ull << (tid >> 7)); rest != 0; rest &= rest - 1) {
-            const int ml = __builtin_ctzll(rest);
-            const int m = m0 + ml, col = nt * (kPTN / 2) + (tid & (kPTN / 2 - 1));
-            if (m >= M || col >= F) continue;
-            const float* x = A + static_cast<long>(m) * K;
-            const uint8_t* gp = B + static_cast<long>(col) * row_bytes;
-            const uint8_t* up = B + static_cast<long>(F + col) * row_bytes;
-            float g = 0.0f, v = 0.0f;
-            for (int k = 0; k < K; ++k) {
-                g = __builtin_fmaf(x[k], decode_row_elem(fmt, gp, k), g);
-                v = __builtin_fmaf(x[k], decode_row_elem(fmt, up, k), v);
-            }
-            C[static_cast<long>(m) * F + col] = silu_f(g) * v;
+    flagged_rows<W>(flagged, A, B, swiglu ? C : out, m0, M, N, K, row_bytes, nt, s_begin, s_end, add, swiglu);
+}
+
+// ---------------------------------------------------------------------------
+// The same product on 128 x 256 tiles, for batches with enough rows that such
+// tiles (and K splits of them) fill the GPU: a wave still decodes its own 32
+// weight rows in registers, but each fragment feeds four MFMAs instead of two,
+// so the decode -- what bounds the kernel above -- costs half per product.  Four
+// m tiles of accumulators leave no room for whole steps of activation fragments,
+// so they are read one 16-column sub-step ahead, and the activations are staged
+// one step at a time, two steps ahead, into a ring of four step tiles, their
+// loads another step ahead; one barrier per step orders the ring (a tile is
+// written in the step after its last read and read from the second step after).
+// What bounds it (1024 x 8192 x K Q4_K, 1.2 us per 64-column step after 12 us to
+// launch, fill and store): the MFMAs alone 0.65 us at the clock that random data
+// leaves them (0.44 on zeros, where the whole step still takes 0.9); without the
+// activation loads 1.0, without their conversion 0.9, without the weight decode
+// 1.0.  Loads a further one or two steps ahead, weights copied through registers,
+// no fences between the phases: 0 to 3% slower.
+constexpr int kWideTM = 128;
+constexpr int kWideStage = kWideTM * kPKS * 2;  // one fp16 activation step tile, bytes
+
+// bytes of a wave's weight area: whole kilobytes for the formats copied straight into LDS, so that
+// every lane of the last copy instruction has a place (the bytes past kAreaBytes repeat its last piece)
+template <class W>
+constexpr int wide_area() {
+    return W::kDmaGroup ? (W::kAreaBytes + 1023) / 1024 * 1024 : W::kAreaBytes;
+}
+
+template <class W>
+constexpr int wide_lds_bytes() {
+    return 4 * kWideStage + (kPThreads / 64) * wide_area<W>() * (W::kDmaGroup ? 2 : 1);
+}
+
+template <class W>
+__global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_wide_kernel(
+    const float* __restrict__ A, const uint8_t* __restrict__ B, float* __restrict__ C, int M, int N, int K,
+    long row_bytes, int MT, int NT, int steps_per_split, int remap, int atomic, float* __restrict__ part, int swiglu) {
+    static_assert(wide_lds_bytes<W>() >= 512 + 64 * kPTN * 4, "half the swiglu epilogue's C tile fits in LDS");
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    int bid = blockIdx.x;
+    if (remap) {  // XCD x (= bid % 8) runs a contiguous run of logical tiles
+        const int per_xcd = gridDim.x >> 3;
+        bid = (bid & 7) * per_xcd + (bid >> 3);
+    }
+    const int mt = bid % MT;  // the m blocks of one weight block are consecutive
+    const int rest = bid / MT;
+    const int nt = rest % NT;
+    const int ksplit = rest / NT;
+    const int s_begin = ksplit * steps_per_split;
+    const int s_end = min(K / kPKS, s_begin + steps_per_split);
+    if (s_begin >= s_end) return;
+    const int nst = s_end - s_begin;  // a multiple of four
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, fr = lane & 31;
+    const int F = N >> 1;  // swiglu: as above
+    const int m0 = mt * kWideTM;
+    const int n0 = swiglu ? (wave >> 2) * F + nt * (kPTN / 2) + 32 * (wave & 3) : nt * kPTN + 32 * wave;
+
+    // activation staging: thread -> columns 4 ap .. 4 ap + 3 of rows ar0 + 32 i
+    const int ap = tid & 15, ar0 = tid >> 4;
+    const float* abase = A + 4 * ap;
+    int arow_off[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) arow_off[i] = min(m0 + ar0 + 32 * i, M - 1) * K;  // M * K < 2^31
+    const int aw = p_off(ar0, ap >> 1) + 8 * (ap & 1);  // row ar0 + 32 i: 4096 i bytes further
+    float amax[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+
+    // weight copy: as above
+    constexpr int kPieces = W::kCopyPieces, kChunks = 32 * kPieces, kLoads = (kChunks + 63) / 64;
+    constexpr int kLoadsA = kLoads > 0 ? kLoads : 1;
+    const int n0c = min(n0, N - 1);
+    const uint8_t* const wbase = B + static_cast<long>(n0c) * row_bytes;
+    int woff[kLoadsA];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        constexpr int kP = kPieces > 0 ? kPieces : 1;
+        const int c = min(64 * i + lane, kChunks - 1);
+        const int r = c / kP;
+        woff[i] = (min(n0 + r, N - 1) - n0c) * static_cast<int>(row_bytes) + 16 * (c % kP);
+    }
+    const int wtoff = (min(n0 + (lane & 31), N - 1) - n0c) * static_cast<int>(row_bytes);
+    char* const warea = lds + 4 * kWideStage + wave * wide_area<W>() * (W::kDmaGroup ? 2 : 1);
+    const char* const wrow = warea + fr * W::kRowBytes;
+    int doff[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = 8 * i + (lane >> 3);
+        const int c = (lane & 7) ^ (r & 7) ^ ((r >> 3) & 1);
+        doff[i] = (min(n0 + r, N - 1) - n0c) * static_cast<int>(row_bytes) + 16 * c;
+    }
+
+    // A-operand fetch offsets of sub-step s (m tile u: 4096 u bytes further)
+    int aoff[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) aoff[s] = p_off(fr, W::chunk(s, h));
+
+    pf16v acc[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[u][i] = 0.0f;
+
+    // Step t (position J = t mod 4): its MFMAs, the decode of step t + 1, the byte reads of step
+    // t + 2, the staging of step t + 2's activations and the loads of step t + 3's.  Loads past the
+    // split's end repeat its last step (in bounds); what they stage is never multiplied.
+    auto step_of = [&](int t) { return s_begin + min(t, nst - 1); };
+    auto step_buf = [&](int t) { return warea + (t % 3) * kPDirectStep; };
+    auto dma = [&](int t) {
+        char* const buf = step_buf(t);
+        const uint8_t* const g = wbase + static_cast<long>(step_of(t)) * (2 * kPKS);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p_dma16(g + doff[i], buf + (kPDirectStep / 4) * i);
+    };
+    typename W::Piece wr[kLoadsA];
+    uint32_t wt = 0;
+    auto load_w = [&](int q) {  // group q's weight bytes, towards LDS
+        if constexpr (W::kDmaGroup) {
+            const uint8_t* g = wbase + W::group_offset(step_of(4 * q));
+            char* const buf = warea + (q & 1) * wide_area<W>();
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i) p_dma16(g + woff[i], buf + 1024 * i);
+        } else if constexpr (!W::kDirect) {
+            const uint8_t* g = wbase + W::group_offset(step_of(4 * q));
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i) wr[i] = W::load_piece(g + woff[i]);
+            if constexpr (W::kTail) wt = W::load_tail(g + wtoff);
         }
-        return;
-    }
-    for (unsigned long long rest = flagged & (0x5555555555555555ull << (tid >> 8)); rest != 0; rest &= rest - 1) {
-        const int ml = __builtin_ctzll(rest);
-        const int m = m0 + ml, nn = nt * kPTN + (tid & 255);
-        if (m >= M || nn >= N) continue;
-        const float* x = A + static_cast<long>(m) * K;
-        const uint8_t* wp = B + static_cast<long>(nn) * row_bytes;
-        float sum = 0.0f;
-        for (int k = s_begin * kPKS; k < s_end * kPKS; ++k) sum = __builtin_fmaf(x[k], decode_row_elem(fmt, wp, k), sum);
-        float* cp = out + static_cast<long>(m) * N + nn;
-        if (add)
-            atomicAdd(cp, sum);
+    };
+    auto write_w = [&]() {
+        if constexpr (!W::kDirect && !W::kDmaGroup) {
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i)
+                if (64 * i + lane < kChunks)
+                    *reinterpret_cast<u32x4*>(warea + 16 * (64 * i + lane)) = W::piece_bytes(wr[i]);
+            if constexpr (W::kTail)
+                if (lane < 32) *reinterpret_cast<uint32_t*>(warea + 32 * W::kRowBytes + 4 * lane) = wt;
+        }
+    };
+    auto load_a = [&](int t, f32x4 (&av)[4]) {
+        const float* p = abase + step_of(t) * kPKS;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) av[i] = ld_f32x4(p + arow_off[i]);
+    };
+    auto stage = [&](char* tile, int i, const f32x4& v) {
+        amax[i] = fmaxf(fmaxf(fmaxf(fmaxf(amax[i], fabsf(v.x)), fabsf(v.y)), fabsf(v.z)), fabsf(v.w));
+        const pf2 p0 = W::kActSwap ? pf2{v.x, v.z} : pf2{v.x, v.y};
+        const pf2 p1 = W::kActSwap ? pf2{v.y, v.w} : pf2{v.z, v.w};
+        const uint32_t lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(p0, ph2));
+        const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(p1, ph2));
+        *reinterpret_cast<pu2*>(tile + aw + 4096 * i) = pu2{lo, hi};
+    };
+    auto afrag = [&](const char* tile, int u, int s) { return *reinterpret_cast<const ph8*>(tile + aoff[s] + 4096 * u); };
+    auto read_w = [&](auto pos, typename W::Frag& f, int t) {  // the lane's bytes of step t, position pos
+        constexpr int P = decltype(pos)::value;
+        if constexpr (W::kDirect)
+            W::read_buf(f, step_buf(t), fr, h);
         else
-            *cp = sum;
+            W::template read<P>(f, wrow + (W::kDmaGroup ? ((t >> 2) & 1) * wide_area<W>() : 0), h);
+    };
+
+    ph8 a0[4], a1[4];          // activation fragments: a sub-step's and the next one's
+    f32x4 av0[4], av1[4];      // activations on the way: steps t + 2 and t + 3
+    typename W::Frag f0, f1;   // bytes of steps t + 1 and t + 2
+    uint32_t b0[4][4], b1[4][4];
+    auto step = [&](auto pos, int t, const uint32_t (&bc)[4][4], uint32_t (&bn)[4][4], const typename W::Frag& fc,
+                    typename W::Frag& fn, f32x4 (&avs)[4], f32x4 (&avl)[4]) {
+        constexpr int J = decltype(pos)::value, Jd = (J + 1) & 3, Jr = (J + 2) & 3;
+        const char* const tile = lds + J * kWideStage;
+        const char* const next = lds + Jd * kWideStage;
+        char* const wtile = lds + Jr * kWideStage;
+        load_a(t + 3, avl);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (J == 0 && !W::kDirect) load_w((t >> 2) + 1);
+        typename W::Consts k;
+        W::template prep<Jd>(fc, k);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            ph8(&ac)[4] = s & 1 ? a1 : a0;
+            ph8(&an)[4] = s & 1 ? a0 : a1;
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                    ac[u], __builtin_bit_cast(ph8, u32x4{bc[s][0], bc[s][1], bc[s][2], bc[s][3]}), acc[u], 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) an[u] = s < 3 ? afrag(tile, u, s < 3 ? s + 1 : 0) : afrag(next, u, 0);
+            if (s == 0) W::template sub<Jd, 0>(fc, k, bn[0]);
+            if (s == 1) W::template sub<Jd, 1>(fc, k, bn[1]);
+            if (s == 2) W::template sub<Jd, 2>(fc, k, bn[2]);
+            if (s == 3) W::template sub<Jd, 3>(fc, k, bn[3]);
+            if (s == W::kReadPhase) {
+                if constexpr (W::kDirect) {
+                    p_wait_vm<4>();  // step t + 2's copy, with step t + 3's activation loads behind it
+                    read_w(std::integral_constant<int, Jr>{}, fn, t + 2);
+                    // step t + 3's copy into the buffer of step t, whose bytes were read two steps ago
+                    dma(t + 3);
+                } else {
+                    if constexpr (Jr == 0) {
+                        // the next group's bytes, requested two steps ago; the eight activation loads of
+                        // this step and the last followed
+                        if constexpr (W::kDmaGroup) p_wait_vm<8>();
+                        write_w();
+                    }
+                    read_w(std::integral_constant<int, Jr>{}, fn, t + 2);
+                }
+            }
+            stage(wtile, s, avs[s]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {  // VALU between the MFMAs, not after them
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+    };
+
+    if constexpr (W::kDirect) {
+        dma(0);
+        dma(1);
+        dma(2);
+    } else {
+        load_w(0);
     }
+    load_a(0, av0);
+    load_a(1, av1);
+    write_w();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        stage(lds, i, av0[i]);
+        stage(lds + kWideStage, i, av1[i]);
+    }
+    load_a(2, av0);
+    if constexpr (W::kDirect || W::kDmaGroup) p_wait_vm<4>();  // the copies
+    read_w(pos_t<0>{}, f0, 0);
+    {
+        typename W::Consts k;
+        W::template prep<0>(f0, k);
+        W::template sub<0, 0>(f0, k, b0[0]);
+        W::template sub<0, 1>(f0, k, b0[1]);
+        W::template sub<0, 2>(f0, k, b0[2]);
+        W::template sub<0, 3>(f0, k, b0[3]);
+    }
+    read_w(pos_t<1>{}, f1, 1);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) a0[u] = afrag(lds, u, 0);
+    for (int t = 0; t < nst; t += 4) {
+        step(pos_t<0>{}, t, b0, b1, f1, f0, av0, av1);
+        step(pos_t<1>{}, t + 1, b1, b0, f0, f1, av1, av0);
+        step(pos_t<2>{}, t + 2, b0, b1, f1, f0, av0, av1);
+        step(pos_t<3>{}, t + 3, b1, b0, f0, f1, av1, av0);
+    }
+    // copies issued for steps past the split's end land before the workgroup's LDS is used again
+    if constexpr (W::kDirect || W::kDmaGroup) p_wait_vm<0>();
+    __syncthreads();
+
+    // rows whose activations left fp16's range take the fp32 path below
+    int* const rowflag = reinterpret_cast<int*>(lds);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float v = amax[i];
+        v = fmaxf(v, __shfl_xor(v, 1));
+        v = fmaxf(v, __shfl_xor(v, 2));
+        v = fmaxf(v, __shfl_xor(v, 4));
+        v = fmaxf(v, __shfl_xor(v, 8));
+        if (ap == 0) rowflag[ar0 + 32 * i] = (v >= kPRowMax || (v > 0.0f && v < kPRowMin)) ? 1 : 0;
+    }
+    __syncthreads();
+    // rows 64 x .. + 63 of the tile, x = 0, 1, as wave-uniform masks, tested in halves (as above)
+    const unsigned long long flagged[2] = {__ballot(rowflag[lane] != 0), __ballot(rowflag[64 + lane] != 0)};
+    const uint32_t fl[4] = {static_cast<uint32_t>(flagged[0]), static_cast<uint32_t>(flagged[0] >> 32),
+                            static_cast<uint32_t>(flagged[1]), static_cast<uint32_t>(flagged[1] >> 32)};
+
+    float* const out = part ? part + static_cast<long>(ksplit) * M * N : C;
+    const bool add = atomic && !part;
+    const int n = n0 + fr;
+    const int mrows = M - m0;
+    if (swiglu) {
+        // 64 rows of the tile at a time through LDS, as above
+        float* const ct = reinterpret_cast<float*>(lds + 512);
+        const int j = tid & (kPTN / 2 - 1), col = nt * (kPTN / 2) + j;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            if (x) __syncthreads();
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    ct[(32 * u + 8 * (i >> 2) + 4 * h + (i & 3)) * kPTN + 32 * wave + fr] = acc[2 * x + u][i];
+            __syncthreads();
+            for (int ml = tid / (kPTN / 2); ml < 64; ml += kPThreads / (kPTN / 2))
+                if (64 * x + ml < mrows && col < F && !(((ml < 32 ? fl[2 * x] : fl[2 * x + 1]) >> (ml & 31)) & 1u))
+                    __builtin_nontemporal_store(silu_f(ct[ml * kPTN + j]) * ct[ml * kPTN + kPTN / 2 + j],
+                                                C + static_cast<long>(m0 + 64 * x + ml) * F + col);
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int ml = 32 * u + 8 * (i >> 2) + 4 * h + (i & 3);
+                if (ml < mrows && n < N && !((fl[u] >> (ml & 31)) & 1u)) {
+                    float* cp = out + static_cast<long>(m0 + ml) * N + n;
+                    if (add)
+                        atomicAdd(cp, acc[u][i]);
+                    else
+                        __builtin_nontemporal_store(acc[u][i], cp);
+                }
+            }
+    }
+
+    // fp32 path for flagged rows: as above
+    for (int x = 0; x < 2; ++x)
+        flagged_rows<W>(flagged[x], A, B, swiglu ? C : out, m0 + 64 * x, M, N, K, row_bytes, nt, s_begin, s_end, add, swiglu);
 }
 
 }  // namespace
@@ -1009,121 +1338,145 @@ bool prefill_supported(int fmt, int M, int N, int K, const void* A, const void* 
 namespace {
 
 // The kernels use more than the default 64 KB of LDS; the limit is raised once per kernel and device.
-template <class W>
-int launch_w(dim3 grid, hipStream_t stream, const float* A, const uint8_t* B, float* C, int M, int N, int K, long rb,
-             int MT, int NT, int sps, int remap, int atomic, float* part, int swiglu = 0) {
+template <class W, bool WIDE>
+int launch_tile(dim3 grid, hipStream_t stream, const float* A, const uint8_t* B, float* C, int M, int N, int K, long rb,
+                int MT, int NT, int sps, int remap, int atomic, float* part, int swiglu) {
     constexpr int kMaxDevices = 64;
-    constexpr int kLds = dev::prefill_lds_bytes<W>();
+    constexpr int kLds = WIDE ? dev::wide_lds_bytes<W>() : dev::prefill_lds_bytes<W>();
+    constexpr auto kernel = WIDE ? &dev::prefill_wide_kernel<W> : &dev::prefill_gemm_kernel<W>;
     static std::atomic<bool> ready[kMaxDevices];
     int devid = 0;
     if (hipGetDevice(&devid) != hipSuccess || devid < 0 || devid >= kMaxDevices) return kFailed;
     if (!ready[devid].load(std::memory_order_acquire)) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&dev::prefill_gemm_kernel<W>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                kLds) != hipSuccess)
             return kFailed;
         ready[devid].store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL(dev::prefill_gemm_kernel<W>, grid, dim3(dev::kPThreads), kLds, stream, A, B, C, M, N, K, rb,
-                       MT, NT, sps, remap, atomic, part, swiglu);
+    hipLaunchKernelGGL(kernel, grid, dim3(dev::kPThreads), kLds, stream, A, B, C, M, N, K, rb, MT, NT, sps, remap,
+                       atomic, part, swiglu);
     return 0;  // the launch's own status is read by the caller
+}
+
+// Tiles and K splits of a product: tm rows per tile (64, or 128: the wide kernel), the k range cut
+// into ks splits of sps steps each (whole groups of four).
+struct PrefillPlan {
+    int tm, ks, sps, MT, NT;
+    long tiles;
+    double us;  // estimated time past what both kernels share
+};
+
+PrefillPlan plan_tiles(int tm, double round_us, double group_us, int M, int N, int K, int NT, long split_floats) {
+    PrefillPlan p;
+    p.tm = tm;
+    p.MT = (M + tm - 1) / tm;
+    p.NT = NT;
+    p.tiles = static_cast<long>(p.MT) * NT;
+    const int nsteps = K / dev::kPKS;
+    int kmax = 1;
+    while (p.tiles * kmax < 256 && nsteps >= 16 * kmax) kmax *= 2;
+    // one workgroup per CU: of the splits up to kmax, the one with the fewest groups of four steps
+    // in sequence on a CU (rounds of 256 workgroups x groups per split), the fewer splits on a tie
+    // (512 x 3072 x 2048: two splits in one round rather than four in two)
+    const long groups = (nsteps + 3) / 4, mn = static_cast<long>(M) * N;
+    p.ks = 1;
+    long best = (p.tiles + 255) / 256 * groups;
+    for (int k = 2; k <= kmax && k * mn <= split_floats; k *= 2) {
+        const long c = (p.tiles * k + 255) / 256 * ((groups + k - 1) / k);
+        if (c < best) best = c, p.ks = k;
+    }
+    int sps = (nsteps + p.ks - 1) / p.ks;
+    p.sps = (sps + 3) / 4 * 4;  // groups of four steps: splits start on one
+    p.ks = (nsteps + p.sps - 1) / p.sps;
+    // partial sums: written and read once more (7 TB/s, mostly from the caches), and a launch to add
+    // them up
+    p.us = (p.tiles * p.ks + 255) / 256 * round_us + best * group_us +
+           (p.ks > 1 ? 2.0 * p.ks * mn * 4 / 7e6 + 2.0 : 0.0);
+    return p;
+}
+
+// The 64-row kernel's plan, which may split K on its own (atomics without a workspace).
+PrefillPlan narrow_plan(int M, int N, int K, int NT) { return plan_tiles(dev::kPTM, 5.0, 3.0, M, N, K, NT, 1L << 62); }
+
+// cols: output columns per tile (kPTN, half of it with the swiglu epilogue); ws_floats: workspace for
+// partial sums (the wide kernel splits K only into one).  A CU takes about 3.0 us for a group of four
+// steps on 64 rows and 4.9 on 128, Q6_K (whose wide form spills) 5.7, and 5 and 9 us to start and store
+// a tile (1343 x 13376 x 256 FP16, one group: 41 us on 64 rows, 51 on 128), so the wide kernel wins
+// where 128-row tiles still fill the GPU or a split does it cheaply: 1024 x 8192 x 2048 Q4_K 64 -> 53 us, FP16 62
+// -> 49, 512 x 16384 x 2048 Q4_K 63 -> 51, 2048 x 3072 x 2048 Q8_0 68 -> 49, Q6_K 80 -> 68, 2048 x 2048
+// x 8192 Q8_0 132 -> 108 (two splits); it loses at 512 x 8192 x 2048 (128 tiles: 33 against 44 us in two splits) and
+// 512 x 2048 x 8192 (eight splits instead of four: 37 against 40).
+PrefillPlan prefill_plan(int fmt, int M, int N, int K, int cols, long ws_floats) {
+    const int NT = (N + cols - 1) / cols;
+    const PrefillPlan a = narrow_plan(M, N, K, NT);
+    // where 64-row tiles already split K, 128-row ones would split it further: 157 x 7516 x 8192 in two splits
+    // 51.8 us, in four of the wide kernel 54.1
+    const PrefillPlan b = plan_tiles(dev::kWideTM, 9.0, fmt == kFmtQ6_K ? 5.7 : 4.9, M, N, K, NT,
+                                     a.ks > 1 ? 0 : std::min<long>(ws_floats, static_cast<long>(dev::kSplitMaxS) * M * N));
+    return b.us < a.us ? b : a;
+}
+
+int launch_plan(int fmt, const PrefillPlan& p, hipStream_t stream, const float* A, const uint8_t* B, float* C, int M,
+                int N, int K, float* part, int swiglu) {
+    const long grid = p.tiles * p.ks;
+    const int remap = grid % 8 == 0 ? 1 : 0, atomic = p.ks > 1 ? 1 : 0;
+    const long rb = row_bytes(fmt, K);
+    const dim3 g(static_cast<unsigned>(grid));
+    auto go = [&](auto w) {
+        using W = decltype(w);
+        return p.tm == dev::kPTM
+                   ? launch_tile<W, false>(g, stream, A, B, C, M, N, K, rb, p.MT, p.NT, p.sps, remap, atomic, part, swiglu)
+                   : launch_tile<W, true>(g, stream, A, B, C, M, N, K, rb, p.MT, p.NT, p.sps, remap, atomic, part, swiglu);
+    };
+    if (fmt == kFmtQ4_K) return go(dev::PQ4K{});
+    if (fmt == kFmtQ6_K) return go(dev::PQ6K{});
+    if (fmt == kFmtQ4_0) return go(dev::PQ4_0{});
+    if (fmt == kFmtQ5_0) return go(dev::PQ5_0{});
+    if (fmt == kFmtF16) return go(dev::PF16{});
+    return go(dev::PQ8_0{});
 }
 
 }  // namespace
 
-// k steps per split and the number of splits: the k range is split over workgroups (whole
-// groups of four steps each) while the tiles alone fill fewer than 256 CUs
-static int prefill_steps_per_split(int M, int N, int K, int* splits) {
-    const long tiles = static_cast<long>((M + dev::kPTM - 1) / dev::kPTM) * ((N + dev::kPTN - 1) / dev::kPTN);
-    const int nsteps = K / dev::kPKS;
-    int kmax = 1;
-    while (tiles * kmax < 256 && nsteps >= 16 * kmax) kmax *= 2;
-    // one workgroup per CU: of the splits up to kmax, the one with the fewest groups of four steps
-    // in sequence on a CU (rounds of 256 workgroups x groups per split), the fewer splits on a tie
-    // (512 x 3072 x 2048: two splits in one round rather than four in two)
-    const long groups = (nsteps + 3) / 4;
-    int ks = 1;
-    long best = groups;
-    for (int k = 2; k <= kmax; k *= 2) {
-        const long cost = (tiles * k + 255) / 256 * ((groups + k - 1) / k);
-        if (cost < best) best = cost, ks = k;
-    }
-    int sps = (nsteps + ks - 1) / ks;
-    sps = (sps + 3) / 4 * 4;  // groups of four steps: splits start on one
-    *splits = (nsteps + sps - 1) / sps;
-    return sps;
+static long split_floats(const PrefillPlan& p, int M, int N) {
+    return p.ks > 1 && p.ks <= dev::kSplitMaxS ? static_cast<long>(p.ks) * M * N : 0;
 }
 
-long prefill_workspace_floats(int M, int N, int K) {
+long prefill_workspace_floats(int fmt, int M, int N, int K, bool least) {
     if (M < 1 || N < 1 || K < 4 * dev::kPKS || K % (4 * dev::kPKS) != 0) return 0;
-    int ks = 1;
-    prefill_steps_per_split(M, N, K, &ks);
-    return ks > 1 && ks <= dev::kSplitMaxS ? static_cast<long>(ks) * M * N : 0;
+    const long a = split_floats(narrow_plan(M, N, K, (N + dev::kPTN - 1) / dev::kPTN), M, N);
+    return least ? a : std::max(a, split_floats(prefill_plan(fmt, M, N, K, dev::kPTN, 1L << 62), M, N));
 }
 
 int launch_prefill_swiglu(int fmt, const float* A, const void* B, float* C, int M, int F, int K, hipStream_t stream) {
     if (F < 1 || !prefill_supported(fmt, M, 2 * F, K, A, B)) return kDeclined;
-    const int MT = (M + dev::kPTM - 1) / dev::kPTM;
-    const int NT = (F + dev::kPTN / 2 - 1) / (dev::kPTN / 2);
-    const long tiles = static_cast<long>(MT) * NT;
+    const PrefillPlan p = prefill_plan(fmt, M, F, K, dev::kPTN / 2, 0);
     // whole k range per workgroup: the epilogue needs finished sums
-    int ks = 1;
-    prefill_steps_per_split(M, 2 * F, K, &ks);
-    if (ks > 1 || tiles > 0x7FFFFFFFL) return kDeclined;
-    const int sps = K / dev::kPKS;
-    const int remap = tiles % 8 == 0 ? 1 : 0;
-    const long rb = row_bytes(fmt, K);
-    const dim3 g(static_cast<unsigned>(tiles));
-    const uint8_t* Bb = static_cast<const uint8_t*>(B);
-    const int N = 2 * F;
-    if (fmt == kFmtQ4_K) return launch_w<dev::PQ4K>(g, stream, A, Bb, C, M, N, K, rb, MT, NT, sps, remap, 0, nullptr, 1);
-    if (fmt == kFmtQ6_K) return launch_w<dev::PQ6K>(g, stream, A, Bb, C, M, N, K, rb, MT, NT, sps, remap, 0, nullptr, 1);
-    if (fmt == kFmtQ4_0) return launch_w<dev::PQ4_0>(g, stream, A, Bb, C, M, N, K, rb, MT, NT, sps, remap, 0, nullptr, 1);
-    if (fmt == kFmtQ5_0) return launch_w<dev::PQ5_0>(g, stream, A, Bb, C, M, N, K, rb, MT, NT, sps, remap, 0, nullptr, 1);
-    if (fmt == kFmtF16) return launch_w<dev::PF16>(g, stream, A, Bb, C, M, N, K, rb, MT, NT, sps, remap, 0, nullptr, 1);
-    return launch_w<dev::PQ8_0>(g, stream, A, Bb, C, M, N, K, rb, MT, NT, sps, remap, 0, nullptr, 1);
+    if (p.ks > 1 || p.tiles > 0x7FFFFFFFL) return kDeclined;
+    return launch_plan(fmt, p, stream, A, static_cast<const uint8_t*>(B), C, M, 2 * F, K, nullptr, 1);
 }
 
 int launch_prefill(int fmt, const float* A, const void* B, float* C, int M, int N, int K, hipStream_t stream, float* ws,
                    long ws_floats, SplitSums* defer, int defer_S) {
     if (defer) defer->S = 0;
-    const int MT = (M + dev::kPTM - 1) / dev::kPTM;
-    const int NT = (N + dev::kPTN - 1) / dev::kPTN;
-    const long tiles = static_cast<long>(MT) * NT;
-    int ks = 1;
-    const int sps = prefill_steps_per_split(M, N, K, &ks);
-    const long grid = tiles * ks;
-    if (grid > 0x7FFFFFFFL) return kDeclined;
-    const int remap = grid % 8 == 0 ? 1 : 0;
-    const int atomic = ks > 1 ? 1 : 0;
+    const long mn = static_cast<long>(M) * N;
+    // partial sums may go to the workspace: its layout and the reduction's 16-byte vectors
+    const bool ws_ok = ws && N % 4 == 0 && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0 &&
+                       (defer || (reinterpret_cast<uintptr_t>(C) & 15u) == 0);
+    const PrefillPlan p = prefill_plan(fmt, M, N, K, dev::kPTN, ws_ok && (!defer || defer_S == 0) ? ws_floats : 0);
+    if (p.tiles * p.ks > 0x7FFFFFFFL) return kDeclined;
+    const int ks = p.ks, atomic = ks > 1 ? 1 : 0;
     // A K split goes, when a workspace holds its partial sums, to plain stores there (split s at
     // ws + s M N), added up in split order by the consumer (defer) or by the reduction kernel:
     // deterministic, and no zero fill; without one, fp32 atomics into a zero-filled C, whose
     // order (and so the last bits) varies.  The atomics are dear: at 512 x 2048 x 8192 Q4_K the
     // kernel storing in their place took 35.3 against 43.0 us (same box), and with the workspace
     // and the reduction launch the product takes 37.3 against 41.1 us.
-    const long mn = static_cast<long>(M) * N;
     float* part = nullptr;
-    if (atomic && ws && ks <= dev::kSplitMaxS && ks * mn <= ws_floats && N % 4 == 0 &&
-        (reinterpret_cast<uintptr_t>(ws) & 15u) == 0 && (defer ? defer_S == 0 || defer_S == ks
-                                                              : (reinterpret_cast<uintptr_t>(C) & 15u) == 0))
+    if (atomic && ws_ok && ks <= dev::kSplitMaxS && ks * mn <= ws_floats && (!defer || defer_S == 0 || defer_S == ks))
         part = ws;
     if (atomic && !part) launch_fill_zero(C, mn, stream);
-    const long rb = row_bytes(fmt, K);
-    const dim3 g(static_cast<unsigned>(grid));
-    const uint8_t* Bb = static_cast<const uint8_t*>(B);
-    int rc;
-    if (fmt == kFmtQ4_K)
-        rc = launch_w<dev::PQ4K>(g, stream, A, Bb, C, M, N, K, rb, MT, NT, sps, remap, atomic, part);
-    else if (fmt == kFmtQ6_K)
-        rc = launch_w<dev::PQ6K>(g, stream, A, Bb, C, M, N, K, rb, MT, NT, sps, remap, atomic, part);
-    else if (fmt == kFmtQ4_0)
-        rc = launch_w<dev::PQ4_0>(g, stream, A, Bb, C, M, N, K, rb, MT, NT, sps, remap, atomic, part);
-    else if (fmt == kFmtQ5_0)
-        rc = launch_w<dev::PQ5_0>(g, stream, A, Bb, C, M, N, K, rb, MT, NT, sps, remap, atomic, part);
-    else if (fmt == kFmtF16)
-        rc = launch_w<dev::PF16>(g, stream, A, Bb, C, M, N, K, rb, MT, NT, sps, remap, atomic, part);
-    else
-        rc = launch_w<dev::PQ8_0>(g, stream, A, Bb, C, M, N, K, rb, MT, NT, sps, remap, atomic, part);
+    const int rc = launch_plan(fmt, p, stream, A, static_cast<const uint8_t*>(B), C, M, N, K, part, 0);
     if (rc != 0 || !part) return rc;
     SplitSums sums;
     sums.part = part;
