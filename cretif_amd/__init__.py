@@ -316,6 +316,11 @@ def _ptr(t):
         return None
     if isinstance(t, int):
         return t
+    try:  # a contiguous device tensor, with as few attribute lookups as tell
+        if t.is_cuda and t.is_contiguous():
+            return t.data_ptr()
+    except AttributeError:
+        pass
     dev = getattr(t, "device", None)
     if dev is None:
         raise TypeError("expected a device tensor or an int address, got %r" % type(t))
@@ -326,11 +331,22 @@ def _ptr(t):
     return t.data_ptr()
 
 
+def _current_stream():
+    """torch's current stream of the current device, as an address.  Building torch's Stream object
+    took 2.9 us of the 8.1 us a small product spends on the host; asking for the address takes 0.3."""
+    import torch
+
+    if not torch.cuda.is_initialized():
+        torch.cuda.init()
+    try:
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    except AttributeError:  # a torch without these
+        return torch.cuda.current_stream().cuda_stream
+
+
 def _stream(stream):
     if stream is None:
-        import torch
-
-        return torch.cuda.current_stream().cuda_stream
+        return _current_stream()
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream  # torch.cuda.Stream
@@ -343,8 +359,10 @@ def _check(status: int):
 
 
 def _mm(name):
+    symbol = "cri_" + name
+
     def fn(A, B, C, M, N, K, stream=None):
-        _check(getattr(lib(), "cri_" + name)(_ptr(A), _ptr(B), _ptr(C), M, N, K, _stream(stream)))
+        _check(getattr(lib(), symbol)(_ptr(A), _ptr(B), _ptr(C), M, N, K, _stream(stream)))
 
     fn.__name__ = name
     fn.__doc__ = "C[M,N] = A[M,K] * dequant(B[N,K])^T (replaces cuinfer::%s)." % name
