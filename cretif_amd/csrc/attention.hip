@@ -396,6 +396,211 @@ __global__ __launch_bounds__(256 / HQ) void decode_attn_split_kernel(const float
     }
 }
 
+// ---- split form, one wave per position tile ------------------------------------
+//
+// The same split, records and arguments for the shapes of long_chunks: chunks of
+// more than two tiles, head_dim above 64, or one query head per KV head.
+//
+// A workgroup is KV head kvh, HQ of its query heads, a chunk of the positions
+// and one query row m (blockIdx.y).  Its four waves take different positions
+// (tiles of 64 / LP of them, wave w: tiles w, w + 4, ...) and each computes all
+// HQ heads on them, so every K and V value passes through the vector memory path
+// of a CU once (above, once per head), and the two tiles a wave has in flight are
+// 16 KB of the cache that no other wave of the workgroup asks for.
+//
+// LP lanes share a position (4 for head_dim up to 64, 8 up to 128): lane r of
+// them holds the dims 4 (r + LP i), i = 0..3, of the query heads, of the tile's
+// K and V rows (16-byte loads) and of the accumulators.  The dot product is
+// summed over the LP lanes, and each position group keeps its own running max,
+// sum and accumulators: the loop has no cross-lane step but that sum.  At the
+// end the groups are rescaled to the wave's max and added (the half-waves and
+// rows of 16 lanes exchange heads, so that row j of a wave ends with head j), and
+// the waves meet in LDS.
+//
+// What bounds it: at short chunks the latency of the first loads and the epilogue
+// (68 partial sums per lane, about 0.5 us); at long ones the bytes in flight.  With
+// the combine, 8191 positions of 8 KV heads: 32 heads of 64 12.3 -> 11.1 us (33.5 MB,
+// 3.0 TB/s), 8 heads of 64 12.2 -> 9.8, 32 heads of 128 20.7 -> 16.8 (67 MB, 4.0 TB/s).
+// Errors against float64 as above (2.0e-7 at 8191 positions).
+constexpr int kSplitWaves = 4;
+
+template <int HQ, int LP>
+__global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_eu(1, 2))) void decode_attn_long_kernel(
+    const float* __restrict__ Q, const float* __restrict__ Kc, const float* __restrict__ Vc, float* __restrict__ ws,
+    int G, int kvd, int D, const int* __restrict__ kv_dev, int kv0, float qscale, int nchunks, int nhq, long ldq) {
+    constexpr int NQ = 4, PT = 64 / LP;  // slices of 4 dims per lane; positions per tile
+    constexpr int LD = 16 * LP + 4;      // floats of a head's part in LDS: acc, max, sum
+    __shared__ __attribute__((aligned(16))) float part[kSplitWaves][4][LD];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = blockIdx.x % nchunks;
+    const int hq = (blockIdx.x / nchunks) % nhq;
+    const int kvh = blockIdx.x / (nchunks * nhq);
+    const int mrow = blockIdx.y;
+    const int H = G * (gridDim.x / (nchunks * nhq));
+    const int p = lane / LP, r = lane % LP;
+    const int h0 = kvh * G + hq * 4;     // first query head of the workgroup
+    const int nh = min(HQ, G - hq * 4);  // and how many it has
+    const float* Qm = Q + mrow * ldq;
+    int dim[NQ];  // clamped into the row: the query's zeros and the stores' checks leave the repeats out
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) dim[i] = min(4 * (r + LP * i), D - 4);
+    f32x4 qv[HQ][NQ];  // requested ahead of the position counter, on which the other addresses depend
+#pragma unroll
+    for (int j = 0; j < HQ; ++j) {
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) qv[j][i] = ld_f32x4(Qm + static_cast<long>(h0 + min(j, nh - 1)) * D + dim[i]);
+    }
+    const int T = (kv_dev ? *kv_dev : 0) + kv0 + mrow;  // positions this row attends to
+    const int Tc = kSplitTile * ((((T + kSplitTile - 1) / kSplitTile) + nchunks - 1) / nchunks);
+    const int t0 = c * Tc, t1 = min(T, t0 + Tc);
+    const float* Kh = Kc + static_cast<long>(kvh) * D;
+    const float* Vh = Vc + static_cast<long>(kvh) * D;
+
+    struct Tile {
+        f32x4 k[NQ], v[NQ];
+    };
+    // this wave's tile n: position t0 + (4 n + wave) PT + p, past the chunk's end its last one
+    auto pos_of = [&](int n) { return t0 + (kSplitWaves * n + wave) * PT + p; };
+    auto load_tile = [&](Tile& t, int n) {
+        const long row = static_cast<long>(min(pos_of(n), t1 - 1)) * kvd;
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) t.k[i] = ld_f32x4(Kh + row + dim[i]);
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) t.v[i] = ld_f32x4(Vh + row + dim[i]);
+    };
+
+    f32x4 acc[HQ][NQ];
+    float m[HQ], l[HQ];
+    auto run_tile = [&](const Tile& t, int n) {
+        const bool live = pos_of(n) < t1;
+#pragma unroll
+        for (int j = 0; j < HQ; ++j) {
+            float s = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) {
+                s = __builtin_fmaf(qv[j][i].x, t.k[i].x, s);
+                s = __builtin_fmaf(qv[j][i].y, t.k[i].y, s);
+                s = __builtin_fmaf(qv[j][i].z, t.k[i].z, s);
+                s = __builtin_fmaf(qv[j][i].w, t.k[i].w, s);
+            }
+            s += dpp<kQuadPerm1032>(s);
+            s += dpp<kQuadPerm2301>(s);
+            if constexpr (LP == 8) s += dpp<0x141>(s);  // row_half_mirror: the other quad of the eight
+            s = live ? s : -INFINITY;
+            const float mn = fmaxf(m[j], s);
+            const float base = mn == -INFINITY ? 0.0f : mn;  // no position yet: factors 0
+            const float cf = __builtin_amdgcn_exp2f(m[j] - base), w = __builtin_amdgcn_exp2f(s - base);
+            m[j] = mn;
+            l[j] = __builtin_fmaf(l[j], cf, w);
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) {
+                acc[j][i].x = __builtin_fmaf(w, t.v[i].x, acc[j][i].x * cf);
+                acc[j][i].y = __builtin_fmaf(w, t.v[i].y, acc[j][i].y * cf);
+                acc[j][i].z = __builtin_fmaf(w, t.v[i].z, acc[j][i].z * cf);
+                acc[j][i].w = __builtin_fmaf(w, t.v[i].w, acc[j][i].w * cf);
+            }
+        }
+    };
+
+    // the wave's tiles: those whose first position lies in the chunk (none in an empty chunk)
+    const int left = t1 - t0 - wave * PT;
+    const int n = left > 0 ? (left + kSplitWaves * PT - 1) / (kSplitWaves * PT) : 0;
+    Tile a, b;
+    if (n > 0) load_tile(a, 0);
+    if (n > 1) load_tile(b, 1);
+    __builtin_amdgcn_sched_barrier(0);  // the tiles' loads are in flight before the query is scaled
+#pragma unroll
+    for (int j = 0; j < HQ; ++j) {
+        m[j] = -INFINITY;
+        l[j] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) {
+            qv[j][i] = 4 * (r + LP * i) < D ? qv[j][i] * qscale : f32x4{0.f, 0.f, 0.f, 0.f};
+            acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    int it = 0;
+    // two tiles in flight; the loads of the last round are clamped to the chunk's last row, so
+    // that they need no branch (behind one, the compiler waits for every load in flight)
+    for (; it + 2 < n; it += 2) {
+        run_tile(a, it);
+        load_tile(a, it + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        run_tile(b, it + 1);
+        load_tile(b, it + 3);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (it < n) run_tile(a, it);
+    if (it + 1 < n) run_tile(b, it + 1);
+
+    // the position groups meet: rescaled to the wave's max of each head (row j of the wave keeps
+    // head j's), then 17 values per head (16 accumulators, the sum) over the lanes of equal r
+    const int row = lane >> 4;
+    auto max_of = [&](int j) { return j < HQ ? m[j < HQ ? j : 0] : -INFINITY; };
+    float M = swap_max16(swap_max32(max_of(0), max_of(2)), swap_max32(max_of(1), max_of(3)));
+    M = fmaxf(M, dpp<0x128>(M));                         // row_ror:8
+    if constexpr (LP == 4) M = fmaxf(M, dpp<0x124>(M));  // row_ror:4
+    float x[4][17];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (j < HQ) {
+            const float mj =
+                __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, M), 16 * j));
+            const float f = mj == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[j < HQ ? j : 0] - mj);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) x[j][e] = acc[j < HQ ? j : 0][e >> 2][e & 3] * f;
+            x[j][16] = l[j < HQ ? j : 0] * f;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 17; ++e) x[j][e] = 0.0f;
+        }
+    }
+    float y[17];
+#pragma unroll
+    for (int e = 0; e < 17; ++e) {
+        // sum of the half-waves: heads 0, 1 in the lower, 2, 3 in the upper; then of the row pairs
+        const float u0 = swap_add32(x[0][e], x[2][e]), u1 = swap_add32(x[1][e], x[3][e]);
+        float v = swap_add16(u0, u1);
+        v += dpp<0x128>(v);                         // row_ror:8
+        if constexpr (LP == 4) v += dpp<0x124>(v);  // row_ror:4
+        y[e] = v;
+    }
+    if ((lane & 15) < LP) {
+        float* o = part[wave][row];
+#pragma unroll
+        for (int i = 0; i < NQ; ++i)
+            *reinterpret_cast<f32x4*>(o + 4 * (r + LP * i)) = f32x4{y[4 * i], y[4 * i + 1], y[4 * i + 2], y[4 * i + 3]};
+        if (r == 0) {
+            o[16 * LP] = M;
+            o[16 * LP + 1] = y[16];
+        }
+    }
+    __syncthreads();
+    // wave j writes the record of head j: max, sum, 2 pad, acc[D] (16-byte aligned)
+    if (wave >= nh) return;
+    float f[kSplitWaves], Mx = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kSplitWaves; ++w) Mx = fmaxf(Mx, part[w][wave][16 * LP]);
+    float L = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kSplitWaves; ++w) {
+        f[w] = Mx == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(part[w][wave][16 * LP] - Mx);
+        L = __builtin_fmaf(f[w], part[w][wave][16 * LP + 1], L);
+    }
+    float* rec = ws + ((static_cast<long>(mrow) * H + h0 + wave) * nchunks + c) * (D + 4);
+#pragma unroll
+    for (int d = lane; d < 16 * LP; d += 64) {
+        float num = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kSplitWaves; ++w) num = __builtin_fmaf(f[w], part[w][wave][d], num);
+        if (d < D) rec[4 + d] = num;
+    }
+    if (lane == 0) {
+        rec[0] = Mx;
+        rec[1] = L;
+    }
+}
+
 // ---- multi-row split form on the fp32 matrix cores (head_dim 64) ---------------
 //
 // For a batch of M query rows (consecutive tokens) one workgroup takes 32
@@ -760,6 +965,35 @@ static void launch_att(bool vec, dim3 grid, hipStream_t stream, const float* Q, 
 }
 
 constexpr int kSplitHeadsPerWave = 1;  // 4 waves per workgroup, one query head each
+
+// Which kernel computes the chunks (microseconds a call with the combine, 40 calls in one graph, one wave per
+// head against one wave per position tile).  Above head_dim 64 the tiles win at every length (32/8 heads
+// of 128: 100 positions 7.65 against 7.19, 2048 10.8 against 10.2, 8191 20.7 against 16.8; a captured decode step
+// of 16 rows, 16/4 heads of 128: 422 against 307), and so they do where a KV head has one query head
+// (8/8 heads of 64: 5.65 against 5.23 at 100, 12.2 against 9.9 at 8191).  With more heads of up to 64 dims their
+// longer epilogue costs 0.4-0.6 us, which chunks of one or two tiles do not give back (32/8 heads: 100
+// positions 5.73 against 6.31, 2048 6.97 against 7.38) and longer ones do (2300 8.21 against 7.97, 4096 9.27 against
+// 9.14, 8191 12.3 against 11.1, 16384 20.0 against 16.3).  Where the length is on the device, a recorded plan
+// meets short rows too, and those heads stay with a wave each.
+static bool long_chunks(int D, int G, const int* kv_dev, long kv_max, int nchunks) {
+    const long tiles = (kv_max + dev::kSplitTile - 1) / dev::kSplitTile;
+    return D > 64 || G == 1 || (!kv_dev && tiles > 2L * nchunks);
+}
+
+// HQ query heads per workgroup (a group of more than four heads: quads of them, the last one
+// possibly shorter)
+template <int HQ>
+static void launch_long(dim3 grid, hipStream_t stream, const float* Q, const float* K, const float* V, float* ws,
+                         int G, int kvd, int D, const int* kv_dev, int kv0, float qscale, int nchunks, int nhq,
+                         long ldq) {
+    if (D <= 64)
+        hipLaunchKernelGGL((dev::decode_attn_long_kernel<HQ, 4>), grid, dim3(64 * dev::kSplitWaves), 0, stream, Q, K,
+                           V, ws, G, kvd, D, kv_dev, kv0, qscale, nchunks, nhq, ldq);
+    else
+        hipLaunchKernelGGL((dev::decode_attn_long_kernel<HQ, 8>), grid, dim3(64 * dev::kSplitWaves), 0, stream, Q, K,
+                           V, ws, G, kvd, D, kv_dev, kv0, qscale, nchunks, nhq, ldq);
+}
+
 constexpr int kMrowMinRows = 4;        // from this many query rows on, head_dim 64 takes the matrix-core form
 
 // Split form: number of chunks (of whole 32-position tiles) that gives ~256
@@ -829,12 +1063,14 @@ int launch_decode_attention_rows(const float* Q, long ldq, const float* K, const
         return 0;
     }
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(rows));
-    if (D <= 64)
+    if (long_chunks(D, G, kv_dev, static_cast<long>(kv0) + rows - 1, nchunks)) {
+        const auto launch = G == 1 ? launch_long<1> : G == 2 ? launch_long<2> : G == 3 ? launch_long<3>
+                                                                                  : launch_long<4>;
+        launch(grid, stream, Q, K, V, ws, G, n_kv_heads * D, D, kv_dev, kv0, qscale, nchunks, nhq, ldq);
+    } else {
         hipLaunchKernelGGL((dev::decode_attn_split_kernel<kSplitHeadsPerWave, 4>), grid, dim3(256 / kSplitHeadsPerWave),
                            0, stream, Q, K, V, ws, G, n_kv_heads * D, D, kv_dev, kv0, qscale, nchunks, nhq, ldq);
-    else
-        hipLaunchKernelGGL((dev::decode_attn_split_kernel<kSplitHeadsPerWave, 8>), grid, dim3(256 / kSplitHeadsPerWave),
-                           0, stream, Q, K, V, ws, G, n_kv_heads * D, D, kv_dev, kv0, qscale, nchunks, nhq, ldq);
+    }
     launch_attention_combine(ws, out, n_heads, rows, D, nchunks, ldo, stream);
     return 0;
 }

@@ -122,5 +122,37 @@ __device__ __forceinline__ float group_sum_t(float v) {
     return v;
 }
 
+// Reductions that halve the number of values.  swap32: lanes below 32 hold (a, a of lane + 32), the others
+// (b of lane - 32, b): v_permlane32_swap exchanges a's upper half with b's lower one.  swap16: the same over
+// pairs of 16-lane rows, even rows a, odd rows b.
+__device__ __forceinline__ f32x2 swap32(float a, float b) {
+    const auto v = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                    false, false);
+    return f32x2{__builtin_bit_cast(float, static_cast<uint32_t>(v[0])),
+                 __builtin_bit_cast(float, static_cast<uint32_t>(v[1]))};
+}
+__device__ __forceinline__ f32x2 swap16(float a, float b) {
+    const auto v = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                    false, false);
+    return f32x2{__builtin_bit_cast(float, static_cast<uint32_t>(v[0])),
+                 __builtin_bit_cast(float, static_cast<uint32_t>(v[1]))};
+}
+__device__ __forceinline__ float swap_add32(float a, float b) {
+    const f32x2 v = swap32(a, b);
+    return v.x + v.y;
+}
+__device__ __forceinline__ float swap_add16(float a, float b) {
+    const f32x2 v = swap16(a, b);
+    return v.x + v.y;
+}
+__device__ __forceinline__ float swap_max32(float a, float b) {
+    const f32x2 v = swap32(a, b);
+    return fmaxf(v.x, v.y);
+}
+__device__ __forceinline__ float swap_max16(float a, float b) {
+    const f32x2 v = swap16(a, b);
+    return fmaxf(v.x, v.y);
+}
+
 }  // namespace dev
 }  // namespace cri
