@@ -4,13 +4,16 @@
 // and 128, on the fp16 matrix cores at fp32 accuracy.
 //
 // Every fp32 operand x is scaled by a power of two into fp16's upper range and
-// taken as two fp16 parts, x = hi + lo to 2^-24 of x, and a product as hi hi +
-// hi lo + lo hi (lo lo is below 2^-24 of it), each exact in fp32 and summed in
-// fp32 with the small ones first.  v_mfma_f32_32x32x16_f16 does 16 times the
-// multiply-adds per cycle of v_mfma_f32_32x32x2_f32, so the three cost 0.19 of
-// the fp32 instruction's cycles.  Against float64 the outputs are closer than
-// those of the fp32 products this replaces (measured beside
-// launch_prompt_attention).
+// taken as two fp16 parts, x = hi + lo, and a product as hi hi + hi lo + lo hi,
+// each exact in fp32 and summed in fp32 with the small ones first.
+// v_mfma_f32_32x32x16_f16 does 16 times the multiply-adds per cycle of
+// v_mfma_f32_32x32x2_f32, so the three cost 0.19 of the fp32 instruction's
+// cycles.  The parts of x are off by at most 2^-23 of x or, for an x below 2^-15
+// of the largest magnitude that shares its scale, 2^-38 of that magnitude (fp16's
+// smallest step); lo lo, left out, is at most 2^-22 of a product and 2^-24 of it
+// on average.  What operands this is enough for, and what happens to the others,
+// stands with kPaSpread.  On N(0, 1) operands the outputs are 1.3 to 4 times
+// closer to float64 than those of the fp32 products (launch_prompt_attention).
 //
 //   * prompt_kv_split_kernel writes the parts of K and V once per call, tile by
 //     tile (32 positions of one KV head, D * 256 bytes), in the order the matrix
@@ -38,12 +41,10 @@
 //     positions are cut into chunks, one (max, sum, acc) record per (row, head,
 //     chunk) for the combine kernel of the decode attention.
 //
-// Parts are good to 2^-24 only for finite values away from the ends of fp32's
-// range: a tile of K or V (or a workgroup's queries) holding an infinity, a NaN or
-// a value of 2^127, or whose largest magnitude is below 2^-100, is flagged, and a
-// workgroup that meets a flag (or V tiles whose largest magnitudes lie more than
-// 2^100 apart) computes its queries with plain fp32 FMAs from the caches instead
-// (attend_slow).
+// A workgroup whose queries or tiles are not of that kind (kPaSpread), or lie at
+// the ends of fp32's range (a tile of K or V, or a query, holding an infinity, a
+// NaN or a value of 2^127, or whose largest magnitude is below 2^-100), computes
+// its queries with plain fp32 FMAs from the caches instead (attend_slow).
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -64,8 +65,20 @@ constexpr int kPaTile = 32;       // positions per tile
 constexpr int kShift = 12;        // log2 of the probabilities' scale
 constexpr float kSlack = 3.0f;    // base-2 headroom of a score over the running maximum
 constexpr uint32_t kPaMax = 0x7F000000u, kPaMin = 0x0D800000u;  // bits of 2^127 and 2^-100
-constexpr int kPaSpread = 100;    // V scales of one workgroup may differ by this many bits
+// The parts' fixed steps must not show beside fp32's rounding (2^-24):
+//   * a score is off by at most D 2^-37 of (largest |q|) (largest |k|), an amount that a score of
+//     fewer or smaller terms may notice; in base 2, where it counts as it is, that is 2^-21 at worst
+//     (aligned signs; 2^-26 as a root of D) while the product is below 2^kPaScore;
+//   * a probability is off by 2^-37 of the largest, so values may be at most 2^kPaSpread apart between the
+//     rows (and dims) a workgroup meets: then the large ones' share is off by 2^-27 of the small ones;
+//   * a value is off by 2^-38 of its tile's largest: 2^-28 of its own row's and dim's largest.
+// Rows and dims of zeros do not count, and dims only in tiles of at least kPaDimRows rows (with fewer, a
+// dim's largest is small by chance).
+constexpr int kPaSpread = 10;
+constexpr int kPaScore = 10;
+constexpr int kPaDimRows = 4;
 constexpr int kPaNoScale = 1 << 20;  // a tile of zeros
+constexpr int kPaZeroExp = 63;       // scale exponent of zeros: as of the smallest magnitudes
 constexpr int kPaXcds = 8;
 
 __host__ __device__ constexpr long pa_tile_bytes(int D) { return static_cast<long>(D) * 256; }
@@ -74,8 +87,8 @@ __host__ __device__ constexpr long pa_tile_bytes(int D) { return static_cast<lon
 struct PaTile {
     float kf;  // 2^-(K scale exponent)
     int ve;    // V scale exponent, kPaNoScale for zeros
+    int vs;    // the scale exponent of V's row or dim of the smallest largest magnitude
     int bad;
-    int pad;
 };
 
 // the two fp16 parts of the pair (a f, b f), f a power of two, each packed in a dword (the lo
@@ -110,6 +123,21 @@ __device__ __forceinline__ uint32_t wave_max_bits(uint32_t v) {
     for (int m = 1; m < 64; m <<= 1) v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), m)));
     return v;
 }
+__device__ __forceinline__ uint32_t wave_min_bits(uint32_t v) {
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) v = min(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), m)));
+    return v;
+}
+// the first N of 2 N values with the lane's bit m clear, the others with it set, each the larger of both lanes'
+template <int N>
+__device__ __forceinline__ void halve_max(uint32_t (&x)[8], int lane, int m) {
+    const bool up = (lane & m) != 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const uint32_t keep = up ? x[N + j] : x[j], give = up ? x[j] : x[N + j];
+        x[j] = max(keep, static_cast<uint32_t>(__shfl_xor(static_cast<int>(give), m)));
+    }
+}
 __device__ __forceinline__ int wave_max_int(int v) {
 #pragma unroll
     for (int m = 1; m < 64; m <<= 1) v = max(v, __shfl_xor(v, m));
@@ -117,8 +145,8 @@ __device__ __forceinline__ int wave_max_int(int v) {
 }
 // true when the parts of values with this largest magnitude are not good to 2^-24
 __device__ __forceinline__ bool out_of_range(uint32_t m) { return m >= kPaMax || (m != 0 && m < kPaMin); }
-// exponent that brings a largest magnitude m (in range) to [2^13, 2^14); 0 for zeros
-__device__ __forceinline__ int scale_exp(uint32_t m) { return m ? 13 + 127 - static_cast<int>(m >> 23) : 0; }
+// exponent that brings a largest magnitude m (in range) to [2^13, 2^14)
+__device__ __forceinline__ int scale_exp(uint32_t m) { return m ? 13 + 127 - static_cast<int>(m >> 23) : kPaZeroExp; }
 __device__ __forceinline__ float pow2(int e) { return __builtin_bit_cast(float, (e + 127) << 23); }  // |e| <= 126
 
 // 16 bytes per lane from global memory into LDS (lane l at byte 16 l of the wave-uniform lds)
@@ -135,6 +163,7 @@ __global__ __launch_bounds__(4 * D) void prompt_kv_split_kernel(const float* __r
                                                                 const int* __restrict__ kv_dev, int kv0, int M) {
     constexpr int kW = 4 * D / 64;
     __shared__ uint32_t red[2][kW];
+    __shared__ uint32_t rows[D / 32][32], cols[2][D];  // largest magnitudes of V's rows and dims, in parts
     const int T = (kv_dev ? *kv_dev : 0) + kv0 + M - 1;
     const int tile = blockIdx.x, kv = blockIdx.y, t0 = tile * kPaTile;
     if (t0 >= T) return;
@@ -162,6 +191,21 @@ __global__ __launch_bounds__(4 * D) void prompt_kv_split_kernel(const float* __r
         km = max(km, absbits(k[e]));
         vm = max(vm, absbits(v[e]));
     }
+    {
+        // a row of V: over the wave's 32 dims; lanes 4 b0 + 2 b1 + b2 of the half-wave end with value e
+        uint32_t x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = absbits(v[e]);
+        halve_max<4>(x, lane, 1);
+        halve_max<2>(x, lane, 2);
+        halve_max<1>(x, lane, 4);
+        x[0] = max(x[0], static_cast<uint32_t>(__shfl_xor(static_cast<int>(x[0]), 8)));
+        x[0] = max(x[0], static_cast<uint32_t>(__shfl_xor(static_cast<int>(x[0]), 16)));
+        const int e = 4 * (lane & 1) + (lane & 2) + ((lane >> 2) & 1);
+        if ((lane & 24) == 0) rows[f >> 1][16 * (f & 1) + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)] = x[0];
+    }
+    vm = max(vm, static_cast<uint32_t>(__shfl_xor(static_cast<int>(vm), 32)));
+    if (lane < 32) cols[f & 1][32 * (f >> 1) + lane] = vm;
     km = wave_max_bits(km);
     vm = wave_max_bits(vm);
     if (lane == 0) {
@@ -189,13 +233,26 @@ __global__ __launch_bounds__(4 * D) void prompt_kv_split_kernel(const float* __r
 #pragma unroll
     for (int q = 0; q < 2; ++q)
         *reinterpret_cast<u32x4*>(out + D * 128 + (q * (D / 16) + f) * 1024 + 16 * lane) = p[q];
-    if (t == 0) {
-        PaTile r;
-        r.kf = pow2(-ke);
-        r.ve = vm ? ve : kPaNoScale;
-        r.bad = bad;
-        r.pad = 0;
-        recs[kv * ntiles + tile] = r;
+    if (f == 0) {
+        uint32_t least = ~0u;  // of the largest magnitudes of V's rows and dims but those of zeros
+        auto take = [&](uint32_t x) { least = x ? min(least, x) : least; };
+        if (T - t0 >= kPaDimRows) {
+#pragma unroll
+            for (int d = lane; d < D; d += 64) take(max(cols[0][d], cols[1][d]));
+        }
+        uint32_t r0 = 0;
+#pragma unroll
+        for (int x = 0; x < D / 32; ++x) r0 = max(r0, rows[x][lane & 31]);
+        take(r0);
+        least = wave_min_bits(least);
+        if (t == 0) {
+            PaTile r;
+            r.kf = pow2(-ke);
+            r.ve = vm ? ve : kPaNoScale;
+            r.vs = scale_exp(least);
+            r.bad = bad;
+            recs[kv * ntiles + tile] = r;
+        }
     }
 }
 
@@ -350,21 +407,24 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
                 qf[1][ks] = p[1];
             }
         }
-        // the records of every tile the workgroup sees: a flag, or V scales too far apart, or queries
-        // out of range take the fp32 path; E is the scale of the accumulators
+        // the records of every tile the workgroup sees: a flag, or magnitudes too far apart, or scores too
+        // large, or queries out of range take the fp32 path; E is the scale of the accumulators
         int E;
         {
             bool slow = out_of_range(qmx);
+            float kfm = 0.0f;  // of the largest |k|
             int lo = -(1 << 20), hi = -(1 << 20);  // -(least exponent), largest exponent
             const PaTile* r = a.recs + static_cast<long>(kvh) * a.ntiles;
             for (int t = first_tile + lane; t * kPaTile < end; t += 64) {
                 slow |= r[t].bad != 0;
-                const int e = r[t].ve;
-                if (e != kPaNoScale) {
-                    lo = max(lo, -e);
-                    hi = max(hi, e);
+                kfm = fmaxf(kfm, r[t].kf);
+                if (r[t].ve != kPaNoScale) {
+                    lo = max(lo, -r[t].ve);
+                    hi = max(hi, r[t].vs);
                 }
             }
+            kfm = wave_max(kfm);
+            slow |= qinv * kfm > pow2(kPaScore - 28);  // the magnitudes are below 2^14 times qinv and kfm
             lo = -wave_max_int(lo);
             hi = wave_max_int(hi);
             E = __builtin_amdgcn_readfirstlane(lo == 1 << 20 ? 0 : lo);

@@ -1,9 +1,9 @@
 """The prompt attention kernel (cri_prefill_attention at head_dim 64 and 128 from 32 rows) at the
 edges of its tiles, query groups and chunks, against the oracle's decode attention row by row.
 
-Bar: 1e-5 normwise, the bar of every fp32 path.  The kernel's own error is the fp16 parts' (2^-24 of
-each operand and of each dropped product, about 4e-7 of a score of magnitude 8) plus fp32 sums over
-the positions, a few 1e-7 in all.
+Bar: 1e-5 normwise, the bar of every fp32 path.  The kernel's own error is the fp16 parts' (at most 2^-23
+of each operand and 2^-22 of a product for the one dropped, a tenth of that in a sum of many) plus fp32
+sums over the positions, a few 1e-7 in all.
 """
 import numpy as np
 import pytest
@@ -58,8 +58,7 @@ def test_matches_oracle(orc, H, Hkv, D, M, pos):
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("what", ["wide", "spread", "tiny_k", "big_q", "zero_v", "peak"])
 def test_ranges(orc, D, what):
-    """Operands of any finite magnitude: tile scales of their own, and the fp32 path where parts
-    would not be exact (V tiles 2^100 apart, a tile or a query below 2^-100, values of 2^127)."""
+    """Operands near the ends of the range, and tiles (that every row sees) of magnitudes far apart."""
     H, Hkv, M, pos = 4, 2, 70, 90
     q, ldq, kc, vc = inputs(M, H, Hkv, D, pos)
     if what == "wide":  # V tiles 2^40 apart, K tiles 2^20 apart (scores stay moderate)
@@ -101,3 +100,68 @@ def test_nonfinite_keys_and_values():
     assert np.isposinf(got[70:, 2:, 5]).all()
     keep = [d for d in range(D) if d != 5]
     assert normwise_rel_err(got[70:, 2:][..., keep], clean[70:, 2:][..., keep]) <= 1e-5
+
+
+def f64(q, kc, vc, rows, H, Hkv, D, pos, scale):
+    """The rows' outputs in float64 and the sums of their terms' magnitudes, [len(rows), H, D] each."""
+    out, mag = np.empty((2, len(rows), H, D))
+    for n, m in enumerate(rows):
+        T = pos + m + 1
+        for h in range(H):
+            g = h // (H // Hkv)
+            v = vc[:T, g].astype(np.float64)
+            s = kc[:T, g].astype(np.float64) @ q[m, h * D:(h + 1) * D].astype(np.float64) * np.float64(scale)
+            p = np.exp(s - s.max())
+            p /= p.sum()
+            out[n, h] = p @ v
+            mag[n, h] = p @ np.abs(v)
+    return out, mag
+
+
+def times(x, at, e):
+    x[at] = (x[at].astype(np.float64) * 2.0 ** e).astype(np.float32)
+
+
+# Magnitudes that differ between positions, or between dims: a row before the first changed position must not
+# notice it, a dim is as good as if it were alone.  Bar: 5e-6 of the sum of an output's terms.  A score is an fp32
+# sum of D products, good to D 2^-24 = 4 to 8e-6 of their magnitudes' sum (about 4) at worst and usually to the root
+# of D in place of D; the softmax passes the error of a score on as a relative one.
+@pytest.mark.parametrize("e", [8, 11, 13, 16, 20, 24, 30, 40, -8, -11, -13, -16, -20, -24, -30, -40])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("what", ["v_tile", "v_row", "k_tile", "k_row", "v_dim", "k_dim", "q_dim", "v_one_key"])
+def test_uneven_magnitudes(what, D, e):
+    H, Hkv, M, pos = 2, 2, 96, 0
+    q, ldq, kc, vc = inputs(M, H, Hkv, D, pos)
+    qh = q.reshape(M, -1, D)
+    scale = np.float32(1.0 / np.sqrt(D))
+    every, first = (slice(None), slice(None), 0), 31
+    if what == "v_tile":
+        times(vc, slice(32, 64), e)
+    elif what == "v_row":
+        times(vc, 31, e)
+    elif what == "k_tile":
+        first = 32
+        times(kc, slice(32, 64), e)
+    elif what == "k_row":
+        times(kc, 31, e)
+    elif what == "v_dim":
+        times(vc, every, e)
+    elif what == "k_dim":  # a score is the sum of a product of a large and a small operand and of the others
+        times(kc, every, e)
+        times(qh, every, -e)
+    elif what == "q_dim":  # the queries' large dim meets keys that are zero there
+        times(qh, every, e)
+        kc[:, :, 0] = 0
+    else:  # value 40 is as large as its weight in row 50 is small
+        for h in range(H):
+            a = qh[50, h].astype(np.float64)
+            kc[40, h] = -abs(e) * np.log(2.0) * np.sqrt(D) * np.sign(a) / np.abs(a).sum()
+        times(vc, 40, abs(e))
+    got = run(q, ldq, kc, vc, M, H, Hkv, D, pos, scale).reshape(M, H, D)
+    assert np.isfinite(got).all()
+    rows = rows_of(M) + [50]
+    if what in ("k_tile", "k_row") and e > 0:  # scores 2^e larger, and the errors of fp32 products with them
+        rows = [m for m in rows if m < first]
+    ref, mag = f64(q, kc, vc, rows, H, Hkv, D, pos, scale)
+    for n, m in enumerate(rows):
+        assert (np.abs(got[m] - ref[n]) <= 5e-6 * mag[n]).all(), (m, np.max(np.abs(got[m] - ref[n]) / mag[n]))
