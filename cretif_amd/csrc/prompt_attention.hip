@@ -41,9 +41,9 @@
 //     positions are cut into chunks, one (max, sum, acc) record per (row, head,
 //     chunk) for the combine kernel of the decode attention.
 //
-// A workgroup whose queries or tiles are not of that kind (kPaSpread), or lie at
+// A workgroup whose queries or tiles are not of that kind (kPaSpread), or lie near
 // the ends of fp32's range (a tile of K or V, or a query, holding an infinity, a
-// NaN or a value of 2^127, or whose largest magnitude is below 2^-100), computes
+// NaN or a value of 2^60, or whose largest magnitude is below 2^-50), computes
 // its queries with plain fp32 FMAs from the caches instead (attend_slow).
 #include <algorithm>
 #include <atomic>
@@ -64,7 +64,10 @@ typedef float paf16 __attribute__((ext_vector_type(16)));
 constexpr int kPaTile = 32;       // positions per tile
 constexpr int kShift = 12;        // log2 of the probabilities' scale
 constexpr float kSlack = 3.0f;    // base-2 headroom of a score over the running maximum
-constexpr uint32_t kPaMax = 0x7F000000u, kPaMin = 0x0D800000u;  // bits of 2^127 and 2^-100
+// bits of 2^60 and 2^-50: scale exponents from -46 to 63, so that the product of two scales, of a tile
+// that is seen or not, and 2^(kShift - a difference of two) are normal numbers (a score's factor of 0 or
+// infinity would meet masked scores of -infinity and scores of 0)
+constexpr uint32_t kPaMax = 0x5D800000u, kPaMin = 0x26800000u;
 // The parts' fixed steps must not show beside fp32's rounding (2^-24):
 //   * a score is off by at most D 2^-37 of (largest |q|) (largest |k|), an amount that a score of
 //     fewer or smaller terms may notice; in base 2, where it counts as it is, that is 2^-21 at worst

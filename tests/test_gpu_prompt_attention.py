@@ -165,3 +165,38 @@ def test_uneven_magnitudes(what, D, e):
     ref, mag = f64(q, kc, vc, rows, H, Hkv, D, pos, scale)
     for n, m in enumerate(rows):
         assert (np.abs(got[m] - ref[n]) <= 5e-6 * mag[n]).all(), (m, np.max(np.abs(got[m] - ref[n]) / mag[n]))
+
+
+# Both operands of the scores small or large together, either side of the range the parts are used in; scores of
+# exactly 0 from large operands; a tile that a query group reads but does not see (rows 0..63 share one at head_dim
+# 64), far from those it sees.  Bar as above.
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("what,a,b", [
+    ("qk", -62, -62), ("qk", -75, -75), ("qk", -49, -49), ("qk", -48, -53), ("qk", -45, -99), ("qk", 58, -58),
+    ("qk", -61, 61), ("zero", 70, 70), ("zero", 50, 50), ("zero", 3, 3), ("later_v", 116, 0), ("later_v", -99, 41),
+    ("later_v", -60, 50), ("later_v", 59, -47), ("later_k", -99, -60), ("later_k", -49, -46)])
+def test_exponents(what, a, b, D):
+    H, Hkv, M, pos = 2, 2, 160, 0
+    q, ldq, kc, vc = inputs(M, H, Hkv, D, pos)
+    qh = q.reshape(M, -1, D)
+    every = slice(None)
+    rows = [m for m in rows_of(M)]
+    if what == "qk":
+        times(qh, every, a)
+        times(kc, every, b)
+    elif what == "zero":
+        times(qh, every, a)
+        times(kc, every, b)
+        qh[:, :, D // 2:] = 0
+        kc[:, :, :D // 2] = 0
+    elif what == "later_v":
+        times(vc, slice(64, None), a)
+        times(vc, slice(64), b)
+    else:
+        times(kc, slice(64, None), a)
+        times(qh, every, b)
+    scale = np.float32(1.0 / np.sqrt(D))
+    got = run(q, ldq, kc, vc, M, H, Hkv, D, pos, scale).reshape(M, H, D)
+    ref, mag = f64(q, kc, vc, rows, H, Hkv, D, pos, scale)
+    for n, m in enumerate(rows):
+        assert (np.abs(got[m] - ref[n]) <= 5e-6 * mag[n]).all(), m
