@@ -43,8 +43,8 @@
 //
 // A workgroup whose queries or tiles are not of that kind (kPaSpread), or lie near
 // the ends of fp32's range (a tile of K or V, or a query, holding an infinity, a
-// NaN or a value of 2^60, or whose largest magnitude is below 2^-50), computes
-// its queries with plain fp32 FMAs from the caches instead (attend_slow).
+// NaN or a value of 2^60, or whose largest magnitude is below 2^-50), takes fp32
+// products from the caches on v_mfma_f32_32x32x2_f32 instead (plain below).
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -270,64 +270,8 @@ struct PromptArgs {
     float* part;  // chunk records otherwise
     long ldq, ldo;
     int kv0, M, G, n_kv, ntiles, nchunks, paired;
-    float qscale;
+    float qscale;  // scale * log2 e: scores are in base 2
 };
-
-// One query (row m, head kvh G + g) over positions [t0, lim) by one wave with fp32 FMAs from the
-// caches: the scores lane by position, then the values lane by dim.
-template <int D>
-__device__ void attend_slow(const PromptArgs& a, int kvh, int m, int g, int c, int t0, int lim) {
-    const int lane = threadIdx.x & 63;
-    const long row = static_cast<long>(a.n_kv) * D;
-    const float* q = a.Q + m * a.ldq + static_cast<long>(kvh * a.G + g) * D;
-    auto score = [&](int t) {
-        const float* k = a.K + t * row + kvh * D;
-        float s = 0.0f;
-#pragma unroll 1
-        for (int d = 0; d < D; ++d) s = __builtin_fmaf(q[d] * a.qscale, k[d], s);
-        return s;
-    };
-    float mx = -INFINITY;
-    bool nan = false;
-    for (int t = t0 + lane; t < lim; t += 64) {
-        const float s = score(t);
-        nan |= s != s;
-        mx = fmaxf(mx, s);
-    }
-    mx = wave_max(mx);
-    if (__any(nan)) mx = NAN;
-    const float base = mx == -INFINITY ? 0.0f : mx;
-    float l = 0.0f, acc[D / 64];
-#pragma unroll
-    for (int j = 0; j < D / 64; ++j) acc[j] = 0.0f;
-    for (int tb = t0; tb < lim; tb += 64) {
-        const int t = tb + lane;
-        const float p = t < lim ? __builtin_amdgcn_exp2f(score(t) - base) : 0.0f;
-        l += p;
-        const int n = min(64, lim - tb);
-#pragma unroll 1
-        for (int u = 0; u < n; ++u) {
-            const float pu = __shfl(p, u);
-#pragma unroll
-            for (int j = 0; j < D / 64; ++j)
-                acc[j] = __builtin_fmaf(pu, a.V[(tb + u) * row + kvh * D + 64 * j + lane], acc[j]);
-        }
-    }
-    l = group_sum_t<6>(l);
-    const int H = a.G * a.n_kv, head = kvh * a.G + g;
-    if (a.out) {
-#pragma unroll
-        for (int j = 0; j < D / 64; ++j) a.out[m * a.ldo + static_cast<long>(head) * D + 64 * j + lane] = acc[j] / l;
-    } else {
-        float* r = a.part + ((static_cast<long>(m) * H + head) * a.nchunks + c) * (D + 4);
-#pragma unroll
-        for (int j = 0; j < D / 64; ++j) r[4 + 64 * j + lane] = acc[j];
-        if (lane == 0) {
-            r[0] = mx;
-            r[1] = l;
-        }
-    }
-}
 
 // floats of one query's record in the merge area (row stride that spreads the banks)
 constexpr int pa_row(int D) { return D + 4; }
@@ -413,8 +357,8 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
         // the records of every tile the workgroup sees: a flag, or magnitudes too far apart, or scores too
         // large, or queries out of range take the fp32 path; E is the scale of the accumulators
         int E;
+        bool slow = out_of_range(qmx);
         {
-            bool slow = out_of_range(qmx);
             float kfm = 0.0f;  // of the largest |k|
             int lo = -(1 << 20), hi = -(1 << 20);  // -(least exponent), largest exponent
             const PaTile* r = a.recs + static_cast<long>(kvh) * a.ntiles;
@@ -432,15 +376,7 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
             hi = wave_max_int(hi);
             E = __builtin_amdgcn_readfirstlane(lo == 1 << 20 ? 0 : lo);
             slow |= hi - lo > kPaSpread;
-            if (__syncthreads_or(slow)) {  // (also: the previous group's merge has been read)
-                for (int x = w; x < 32 * QB; x += kWaves) {
-                    const int qq = grp * 32 * QB + x;
-                    if (qq >= nq) break;
-                    const int m = qq / a.G;
-                    attend_slow<D>(a, kvh, m, qq - m * a.G, c, t0, min(Tb + m, t1));
-                }
-                return;
-            }
+            slow = __syncthreads_or(slow);  // (also: the previous group's merge has been read)
         }
 
         // the K or V half of stage st's tiles into buffer st & 1; the waves share the copies
@@ -546,6 +482,114 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
         };
         const char* const mine = lds + kw * kHalf + 16 * lane;
         int tb = t0 + kw * kPaTile;
+        // The same tiles with fp32 products, in the same transposed layout: the n-th instruction of S^T takes dim
+        // 8 (n >> 2) + 4 h + (n & 3) from lane (i, h) for key i and query i, the n-th of a dim block of O^T position
+        // 8 (n >> 2) + 4 h + (n & 3), whose probability the lane holds in its n-th score.  Bound by the matrix
+        // instructions and, its loads hidden by the SIMD's other wave only, their latency: every query of 2048 rows,
+        // 32/8 heads of 64, 249 us (the five launches over materialized scores 591, one query at a time on scalar
+        // FMAs 18300); heads of 128 481 (768, 33500); 64 rows 17 (32, 262).
+        auto plain = [&]() {
+            const long row = static_cast<long>(a.n_kv) * D;
+            const float *const Kh = a.K + kvh * D + 4 * h, *const Vh = a.V + kvh * D;
+            const float* const qp = a.Q + qm * a.ldq + static_cast<long>(kvh * a.G + qg) * D + 4 * h;
+            float* const ps = reinterpret_cast<float*>(lds) + w * 2048;  // [32 positions][32 queries], then [..][dims]
+            static_assert(pa_lds_bytes<D, QB, KS>() >= kWaves * 8192);
+            const int hi = q0 < nq ? min(Tb + min(q0 + 31, nq - 1) / a.G, t1) : t0;  // the wave's last limit
+            for (; tb < hi; tb += kStagePos) {
+                const float* const kp = Kh + min(tb + i, Tmax - 1) * row;
+                paf16 sa, sb;  // two chains
+#pragma unroll
+                for (int v = 0; v < 16; ++v) sa[v] = sb[v] = 0.0f;
+#pragma unroll
+                for (int c = 0; c < D / 64; ++c) {
+                    // (the query is read again for every tile: at head_dim 128 there is no room to keep it)
+                    if constexpr (D > 64) asm volatile("" ::: "memory");
+                    f32x4 k[8], qv[8];
+#pragma unroll
+                    for (int n = 0; n < 8; ++n) k[n] = ld_f32x4(kp + 64 * c + 8 * n);
+#pragma unroll
+                    for (int n = 0; n < 8; ++n) qv[n] = ld_f32x4(qp + 64 * c + 8 * n);
+#pragma unroll
+                    for (int n = 0; n < 8; ++n) {
+                        sa = __builtin_amdgcn_mfma_f32_32x32x2f32(k[n].x, qv[n].x, sa, 0, 0, 0);
+                        sb = __builtin_amdgcn_mfma_f32_32x32x2f32(k[n].y, qv[n].y, sb, 0, 0, 0);
+                        sa = __builtin_amdgcn_mfma_f32_32x32x2f32(k[n].z, qv[n].z, sa, 0, 0, 0);
+                        sb = __builtin_amdgcn_mfma_f32_32x32x2f32(k[n].w, qv[n].w, sb, 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                float p[16], tmax = -INFINITY;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    p[v] = tb + 8 * (v >> 2) + 4 * h + (v & 3) < lim ? (sa[v] + sb[v]) * a.qscale : -INFINITY;
+                    tmax = fmaxf(tmax, p[v]);
+                }
+                const float mnew = fmaxf(mx, fmaxf(tmax, shfl_xor32(tmax)));
+                const float base = mnew == -INFINITY ? 0.0f : mnew;
+                const float cf = __builtin_amdgcn_exp2f(mx - base);
+                mx = mnew;
+                l *= cf;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    p[v] = __builtin_amdgcn_exp2f(p[v] - base);
+                    l += p[v];
+                }
+#pragma unroll
+                for (int d = 0; d < kDb; ++d) o[d] *= cf;
+#pragma unroll
+                for (int d0 = 0; d0 < kDb; d0 += 2) {
+                    float x[2][16];
+                    bool odd = false;
+#pragma unroll
+                    for (int n = 0; n < 16; ++n) {
+                        const float* const vp =
+                            Vh + min(tb + 8 * (n >> 2) + 4 * h + (n & 3), Tmax - 1) * row + 32 * d0 + i;
+#pragma unroll
+                        for (int d = 0; d < 2; ++d) {
+                            x[d][n] = vp[32 * d];
+                            odd |= absbits(x[d][n]) >= 0x7F800000u;
+                        }
+                    }
+                    if (tb + kPaTile > lim_lo && __any(odd)) {
+                        // an infinite or NaN value that not every query sees: times the probability 0 of those
+                        // that do not, it would reach them
+#pragma unroll
+                        for (int d = 0; d < 2; ++d) {
+#pragma unroll
+                            for (int v = 0; v < 16; ++v) {
+                                ps[32 * (8 * (v >> 2) + 4 * h + (v & 3)) + i] = p[v];
+                                ps[32 * (32 + 8 * (v >> 2) + 4 * h + (v & 3)) + i] = x[d][v];
+                            }
+                            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                            __builtin_amdgcn_wave_barrier();
+#pragma unroll 4
+                            for (int u = 0; u < kPaTile; ++u) {
+                                const float pu = ps[32 * u + i];
+                                const uint32_t seen = tb + u < lim ? ~0u : 0u;  // (a select would become branches)
+#pragma unroll
+                                for (int v = 0; v < 4; ++v) {
+                                    const u32x4 y =
+                                        *reinterpret_cast<const u32x4*>(ps + 32 * (32 + u) + 8 * v + 4 * h) & seen;
+                                    const f32x4 z = __builtin_bit_cast(f32x4, y);
+#pragma unroll
+                                    for (int e = 0; e < 4; ++e)
+                                        o[d0 + d][4 * v + e] = __builtin_fmaf(pu, z[e], o[d0 + d][4 * v + e]);
+                                }
+                            }
+                            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                            __builtin_amdgcn_wave_barrier();
+                        }
+                    } else {
+#pragma unroll
+                        for (int n = 0; n < 16; ++n)
+#pragma unroll
+                            for (int d = 0; d < 2; ++d)
+                                o[d0 + d] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[d][n], p[n], o[d0 + d], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        };
         // stage st (position J = st & 1 of the buffers); r: its tile's record, the next one's when it returns
         auto stage = [&](int st, auto pos, float& kf, int& ve, paf16& s, paf16& sn) {
             constexpr int J = decltype(pos)::value;
@@ -565,7 +609,9 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
             ve = ven;
             tb += kStagePos;
         };
-        if (nst > 0) {
+        if (slow) {
+            plain();
+        } else if (nst > 0) {
             paf16 s0, s1;
             float kf = recs[rec_of(0)].kf;
             int ve = recs[rec_of(0)].ve;
@@ -626,8 +672,8 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
                         for (int e = 0; e < 4; ++e) o[d][4 * v + e] = __builtin_fmaf(f, y[e], o[d][4 * v + e]);
                     }
             }
-            // the accumulators hold 2^(kShift + E) times the sums (two factors: E + kShift may be 125)
-            const float back = pow2(-E) * pow2(-kShift);
+            // the accumulators hold 2^(kShift + E) times the sums, or the sums
+            const float back = slow ? 1.0f : pow2(-E - kShift);
             const int head = kvh * a.G + qg;
             float* dst;
             if (a.out) {

@@ -200,3 +200,33 @@ def test_exponents(what, a, b, D):
     ref, mag = f64(q, kc, vc, rows, H, Hkv, D, pos, scale)
     for n, m in enumerate(rows):
         assert (np.abs(got[m] - ref[n]) <= 5e-6 * mag[n]).all(), m
+
+
+# Values too small for the parts: every workgroup takes the fp32 products, in all the forms of test_matches_oracle.  A
+# NaN key and an infinite value reach exactly the rows that see them.
+@pytest.mark.parametrize("H,Hkv,D,M,pos", [
+    (1, 1, 64, 32, 0), (7, 1, 64, 33, 31), (3, 1, 128, 37, 3), (8, 8, 128, 65, 0), (32, 8, 64, 64, 959),
+    (4, 1, 128, 300, 700), (32, 8, 64, 513, 0), (8, 8, 64, 1000, 24), (32, 8, 64, 1025, 0), (32, 8, 128, 1030, 5)])
+def test_fp32_products(H, Hkv, D, M, pos):
+    q, ldq, kc, vc = inputs(M, H, Hkv, D, pos)
+    times(vc, slice(None), -60)
+    t_inf, t_nan = pos + M // 2, pos + M - 5
+    vc[t_inf, 0, 5] = np.inf
+    kc[t_nan, Hkv - 1, 3] = np.nan
+    scale = np.float32(1.0 / np.sqrt(D))
+    got = run(q, ldq, kc, vc, M, H, Hkv, D, pos, scale).reshape(M, H, D)
+    rows = sorted({*rows_of(M), M // 2 - 1, M - 6, M - 5})
+    vc[t_inf, 0, 5] = 0
+    kc[t_nan, Hkv - 1, 3] = 0
+    ref, mag = f64(q, kc, vc, rows, H, Hkv, D, pos, scale)
+    G = H // Hkv
+    for n, m in enumerate(rows):
+        for h in range(H):
+            if pos + m >= t_nan and h // G == Hkv - 1:
+                assert np.isnan(got[m, h]).all(), (m, h)
+                continue
+            dims = np.ones(D, bool)
+            if pos + m >= t_inf and h // G == 0:
+                dims[5] = False
+                assert not np.isfinite(got[m, h, 5]), (m, h)  # NaN where the records of chunks are merged
+            assert (np.abs(got[m, h] - ref[n, h]) <= 5e-6 * mag[n, h])[dims].all(), (m, h)
