@@ -121,25 +121,33 @@ __device__ __forceinline__ paf16 mma(const u32x4& a, const u32x4& b, const paf16
 
 // magnitudes are compared as bit patterns, which order as the floats do with NaN above infinity
 __device__ __forceinline__ uint32_t absbits(float x) { return __builtin_bit_cast(uint32_t, x) & 0x7FFFFFFFu; }
+// Reductions on the VALU alone (a __shfl_xor is a trip through the LDS pipe): quad permutations, rotations of
+// 16-lane rows, and exchanges of rows and half-waves.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_bits(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), CTRL, 0xF, 0xF, false));
+}
+constexpr int kRowRor4 = 0x124, kRowRor8 = 0x128;
+__device__ __forceinline__ uint32_t max32(uint32_t v) {  // with lane ^ 32
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return max(static_cast<uint32_t>(r[0]), static_cast<uint32_t>(r[1]));
+}
+// even 16-lane rows: the larger of a and lane + 16's a; odd ones: of b and lane - 16's b
+__device__ __forceinline__ uint32_t max16(uint32_t a, uint32_t b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    return max(static_cast<uint32_t>(r[0]), static_cast<uint32_t>(r[1]));
+}
 __device__ __forceinline__ uint32_t wave_max_bits(uint32_t v) {
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), m)));
-    return v;
+    v = max(v, dpp_bits<kQuadPerm1032>(v));
+    v = max(v, dpp_bits<kQuadPerm2301>(v));
+    v = max(v, dpp_bits<kRowRor4>(v));
+    v = max(v, dpp_bits<kRowRor8>(v));
+    return max32(max16(v, v));
 }
-__device__ __forceinline__ uint32_t wave_min_bits(uint32_t v) {
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) v = min(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), m)));
-    return v;
-}
-// the first N of 2 N values with the lane's bit m clear, the others with it set, each the larger of both lanes'
-template <int N>
-__device__ __forceinline__ void halve_max(uint32_t (&x)[8], int lane, int m) {
-    const bool up = (lane & m) != 0;
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-        const uint32_t keep = up ? x[N + j] : x[j], give = up ? x[j] : x[N + j];
-        x[j] = max(keep, static_cast<uint32_t>(__shfl_xor(static_cast<int>(give), m)));
-    }
+// the larger of the lanes' a (bit m of the lane clear) or b (set), CTRL exchanging lanes that differ in m alone
+template <int CTRL>
+__device__ __forceinline__ uint32_t halve_max(uint32_t a, uint32_t b, bool set) {
+    return max(set ? b : a, dpp_bits<CTRL>(set ? a : b));
 }
 __device__ __forceinline__ int wave_max_int(int v) {
 #pragma unroll
@@ -195,19 +203,20 @@ __global__ __launch_bounds__(4 * D) void prompt_kv_split_kernel(const float* __r
         vm = max(vm, absbits(v[e]));
     }
     {
-        // a row of V: over the wave's 32 dims; lanes 4 b0 + 2 b1 + b2 of the half-wave end with value e
-        uint32_t x[8];
+        // a row of V: over the wave's 32 dims; the lanes end with the value e of their bits 4, 0 and 1
+        uint32_t x[4];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = absbits(v[e]);
-        halve_max<4>(x, lane, 1);
-        halve_max<2>(x, lane, 2);
-        halve_max<1>(x, lane, 4);
-        x[0] = max(x[0], static_cast<uint32_t>(__shfl_xor(static_cast<int>(x[0]), 8)));
-        x[0] = max(x[0], static_cast<uint32_t>(__shfl_xor(static_cast<int>(x[0]), 16)));
-        const int e = 4 * (lane & 1) + (lane & 2) + ((lane >> 2) & 1);
-        if ((lane & 24) == 0) rows[f >> 1][16 * (f & 1) + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)] = x[0];
+        for (int e = 0; e < 4; ++e) x[e] = max16(absbits(v[e]), absbits(v[4 + e]));
+        x[0] = halve_max<kQuadPerm1032>(x[0], x[2], lane & 1);
+        x[1] = halve_max<kQuadPerm1032>(x[1], x[3], lane & 1);
+        x[0] = halve_max<kQuadPerm2301>(x[0], x[1], lane & 2);
+        x[0] = max(x[0], dpp_bits<kRowRor8>(x[0]));
+        x[0] = max(x[0], dpp_bits<kRowRor4>(x[0]));
+        if ((lane & 12) == 0)  // e = 4 (bit 4) + 2 (bit 0) + (bit 1)
+            rows[f >> 1][16 * (f & 1) + 8 * ((lane >> 4) & 1) + 4 * (lane >> 5) + 2 * (lane & 1) +
+                         ((lane >> 1) & 1)] = x[0];
     }
-    vm = max(vm, static_cast<uint32_t>(__shfl_xor(static_cast<int>(vm), 32)));
+    vm = max32(vm);
     if (lane < 32) cols[f & 1][32 * (f >> 1) + lane] = vm;
     km = wave_max_bits(km);
     vm = wave_max_bits(vm);
@@ -237,8 +246,8 @@ __global__ __launch_bounds__(4 * D) void prompt_kv_split_kernel(const float* __r
     for (int q = 0; q < 2; ++q)
         *reinterpret_cast<u32x4*>(out + D * 128 + (q * (D / 16) + f) * 1024 + 16 * lane) = p[q];
     if (f == 0) {
-        uint32_t least = ~0u;  // of the largest magnitudes of V's rows and dims but those of zeros
-        auto take = [&](uint32_t x) { least = x ? min(least, x) : least; };
+        uint32_t inv = 0;  // ~(the least of the largest magnitudes of V's rows and dims but those of zeros)
+        auto take = [&](uint32_t x) { inv = max(inv, x ? ~x : 0u); };
         if (T - t0 >= kPaDimRows) {
 #pragma unroll
             for (int d = lane; d < D; d += 64) take(max(cols[0][d], cols[1][d]));
@@ -247,12 +256,12 @@ __global__ __launch_bounds__(4 * D) void prompt_kv_split_kernel(const float* __r
 #pragma unroll
         for (int x = 0; x < D / 32; ++x) r0 = max(r0, rows[x][lane & 31]);
         take(r0);
-        least = wave_min_bits(least);
+        inv = wave_max_bits(inv);
         if (t == 0) {
             PaTile r;
             r.kf = pow2(-ke);
             r.ve = vm ? ve : kPaNoScale;
-            r.vs = scale_exp(least);
+            r.vs = scale_exp(~inv);
             r.bad = bad;
             recs[kv * ntiles + tile] = r;
         }
