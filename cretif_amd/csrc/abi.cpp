@@ -123,6 +123,12 @@ int dequant_impl(int fmt, const void* src, float* dst, int n_blocks, hipStream_t
 
 void cri_internal_set_error(const char* msg) { g_last_error = msg; }
 
+// rows per tile of the prefill GEMM for a shape it takes (64 or 128), with a workspace of that many bytes (0: none) or
+// the SiLU * up epilogue (N: its output columns): for tests that mean one of the two kernels
+extern "C" int cri_internal_prefill_tile_rows(int format, int M, int N, int K, long long workspace_bytes, int swiglu) {
+    return cri::detail::prefill_tile_rows(format, M, N, K, static_cast<long>(workspace_bytes / 4), swiglu != 0);
+}
+
 namespace {
 int fill_zero(float* C, long n, hipStream_t stream, const char* fn) {
     clear_pending_error();

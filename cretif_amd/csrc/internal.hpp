@@ -184,6 +184,8 @@ int launch_prefill_swiglu(int fmt, const float* A, const void* B, float* C, int 
 // those of the 64-row kernel, without which the split it makes on its own would take atomics (the
 // 128-row kernel's split is only made where a workspace holds it)
 long prefill_workspace_floats(int fmt, int M, int N, int K, bool least);
+// rows per tile (64 or 128) that launch_prefill, or launch_prefill_swiglu with F = N, takes for this shape
+int prefill_tile_rows(int fmt, int M, int N, int K, long ws_floats, bool swiglu);
 // C = the S partial sums of p added in split order (times p's RMSNorm row factor); M N % 4 == 0,
 // C and p.part 16-byte aligned, p.stride % 4 == 0 (mfma_skinny.hip)
 int launch_split_reduce(const SplitSums& p, float* C, int M, hipStream_t stream);

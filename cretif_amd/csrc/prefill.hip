@@ -1448,6 +1448,10 @@ long prefill_workspace_floats(int fmt, int M, int N, int K, bool least) {
     return least ? a : std::max(a, split_floats(prefill_plan(fmt, M, N, K, dev::kPTN, 1L << 62), M, N));
 }
 
+int prefill_tile_rows(int fmt, int M, int N, int K, long ws_floats, bool swiglu) {
+    return prefill_plan(fmt, M, N, K, swiglu ? dev::kPTN / 2 : dev::kPTN, swiglu ? 0 : ws_floats).tm;
+}
+
 int launch_prefill_swiglu(int fmt, const float* A, const void* B, float* C, int M, int F, int K, hipStream_t stream) {
     if (F < 1 || !prefill_supported(fmt, M, 2 * F, K, A, B)) return kDeclined;
     const PrefillPlan p = prefill_plan(fmt, M, F, K, dev::kPTN / 2, 0);

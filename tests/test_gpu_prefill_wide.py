@@ -18,8 +18,18 @@ def tiled(fmt, N, K, seed, rows=640):
     return np.ascontiguousarray(np.resize(np.arange(rows), N)), w
 
 
-def product(fmt, A, w, order, N, K, ws=None):
+def tile_rows(fmt, M, N, K, ws_bytes=0, swiglu=False):
+    """The rows of the prefill GEMM's tiles for this call: 128 is the kernel of this file."""
+    import ctypes
+
+    f = cri.lib().cri_internal_prefill_tile_rows
+    f.argtypes = [ctypes.c_int] * 4 + [ctypes.c_longlong, ctypes.c_int]
+    return f(cri.FORMAT_IDS[fmt], M, N, K, ws_bytes, swiglu)
+
+
+def product(fmt, A, w, order, N, K, ws=None, rows=128):
     M = A.shape[0]
+    assert tile_rows(fmt, M, N, K, 0 if ws is None else 4 * ws.numel()) == rows
     C = torch.full((M, N), float("nan"), device="cuda")
     B = dev(w)[torch.from_numpy(order).cuda()].contiguous()
     if ws is None:
@@ -31,7 +41,7 @@ def product(fmt, A, w, order, N, K, ws=None):
 
 # one to five groups of four steps; one and three row tiles with ragged last ones; a ragged last column tile
 @pytest.mark.parametrize("fmt", FMTS)
-@pytest.mark.parametrize("M,N,K", [(65, 65533, 256), (128, 65536, 768), (300, 21800, 512), (129, 32768, 1280)])
+@pytest.mark.parametrize("M,N,K", [(65, 65533, 256), (128, 65536, 768), (300, 21755, 512), (129, 32768, 1280)])
 def test_matches_oracle(orc, fmt, M, N, K):
     rng = np.random.default_rng(M + K)
     A = rng.standard_normal((M, K)).astype(np.float32)
@@ -68,7 +78,7 @@ def test_exact_integers(orc, fmt):
 @pytest.mark.parametrize("fmt", ["q4_k", "q8_0", "q4_0", "q5_0", "fp16"])
 def test_workspace_split(orc, fmt):
     """A long prompt's down projection: K in two splits through the workspace (the same bits on every
-    call); without a workspace, or with one too small, or unaligned, the unsplit kernel."""
+    call); without a workspace, or with one too small, or unaligned, the unsplit 64-row kernel."""
     M, N, K = 2048, 2048, 8192
     rng = np.random.default_rng(9)
     A = rng.standard_normal((M, K)).astype(np.float32)
@@ -81,7 +91,7 @@ def test_workspace_split(orc, fmt):
     rows = [0, 63, 64, 127, 128, 1000, 2047]
     ref = orc.matmul_quant(fmt, A[rows], w.reshape(-1), w.shape[0], K)[:, order]
     assert normwise_rel_err(a[rows], ref) <= PREFILL_TOL
-    b = product(fmt, A, w, order, N, K)
+    b = product(fmt, A, w, order, N, K, rows=64)
     assert normwise_rel_err(a, b) <= 1e-5  # the order of fp32 sums
     C = torch.full((M, N), float("nan"), device="cuda")
     B = dev(w)[torch.from_numpy(order).cuda()].contiguous()
@@ -125,5 +135,6 @@ def test_prompt_swiglu(orc, norm):
     dec.set_position(pos)
     dec.forward(ids, M, a)
     got = a.cpu().numpy()
+    assert tile_rows("fp16", M, 32768, 256, swiglu=True) == 128
     ref, _ = orc.decode_step(m, list(ids.cpu().numpy()), pos, [k.copy() for k in kc], [v.copy() for v in vc])
     assert np.isfinite(got).all() and normwise_rel_err(got, ref) <= PREFILL_TOL
