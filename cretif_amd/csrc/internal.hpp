@@ -173,9 +173,10 @@ bool prefill_supported(int fmt, int M, int N, int K, const void* A, const void* 
 // takes, 0 any), else added up into C (16-byte aligned) in split order by a second launch.
 int launch_prefill(int fmt, const float* A, const void* B, float* C, int M, int N, int K, hipStream_t stream,
                    float* ws = nullptr, long ws_floats = 0, SplitSums* defer = nullptr, int defer_S = 0);
-// K splits of the prefill GEMM are chosen so that tiles x splits < 512; so at most this many
-// partial-sum floats (512 tiles of 128 x 256); splits past 16 take the atomics
-constexpr long kPrefillSplitFloats = 512L * 128 * 256;
+// the most partial-sum floats of a K split that goes to a workspace: a split count k is only taken
+// over k / 2 where tiles x k fit one round of 256 workgroups (with more rounds the groups in
+// sequence are at least as many), so 256 tiles of 128 x 256; splits past 16 take the atomics
+constexpr long kPrefillSplitFloats = 256L * 128 * 256;
 // C[M, F] = SiLU(A gate^T) * (A up^T) for a stacked gate/up matrix B of 2F rows (gate first), the
 // product and the elementwise step in one launch (the SiLU * up of the separate kernel, bit for
 // bit); kDeclined where the tiles would need a K split (short prompts) or the kernel does not apply

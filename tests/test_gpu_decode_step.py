@@ -564,6 +564,25 @@ def test_prompt_row_blocks_nan_cache_and_replay(orc, head_dim):
     assert normwise_rel_err(b.cpu().numpy(), eager) <= 1e-5
 
 
+def test_prompt_workspace_size():
+    # the split workspace is sized by what a plan can use, 256 tiles of 128 x 256 floats (34 MB), not by twice that;
+    # the rest of so small a decoder is a few MB
+    fmts = ("q8_0", "q4_0", "q5_0", "q4_k", "q6_k", "fp16")
+    most = max(cri.matmul_workspace_bytes(f, M, N, K) for f in fmts for M in (17, 63, 65, 128, 200, 512, 777, 2048)
+               for N in (1, 64, 260, 1000, 2048, 3072, 4096, 8192, 16384) for K in (256, 1024, 2048, 4352, 8192, 16384))
+    assert 200 * 128 * 256 * 4 < most <= 256 * 128 * 256 * 4
+    m = make_model(1, dim=256, n_heads=4, n_kv_heads=2, head_dim=64, ffn=256, vocab=64, seed=3,
+                   fmts={n: "fp16" for n in ("q", "k", "v", "o", "gate", "up", "down")}, tok="q8_0", lm="fp16",
+                   big_tables=False)
+    make_decoder(m, max_seq=64, max_batch=17)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    dec = make_decoder(m, max_seq=64, max_batch=17)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < 48 << 20
+    del dec
+
+
 @pytest.mark.parametrize("ffn", [1056, 1024])
 def test_prompt_swiglu_partial_tile(orc, ffn):
     # the fused gate/up + SiLU * up launch covers 128 output columns per tile: an FFN width that is
