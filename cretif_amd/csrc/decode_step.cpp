@@ -29,8 +29,9 @@ namespace {
 // Batches up to this many tokens take the fused RMSNorm / SwiGLU prologues.
 constexpr int kFusedMaxBatch = 16;
 // Larger batches (a prompt) run attention on the prompt kernel (from kPromptAttnMinRows rows at
-// head_dim 64 and 128), below that at head_dim 64 on the multi-row split kernel, otherwise through batched_matmul_gqa in row blocks of cri::detail::kPromptRows rows (the scores workspace
-// holds n_heads x that x max_seq_len floats).
+// head_dim 64 and 128), below that at head_dim 64 on the multi-row split kernel, otherwise through
+// batched_matmul_gqa in row blocks of cri::detail::kPromptRows rows (the scores workspace holds
+// n_heads x that x max_seq_len floats).
 using cri::detail::kPromptRows;
 
 int round4(int n) { return (n + 3) / 4 * 4; }
@@ -180,7 +181,8 @@ DecodeStep::DecodeStep(const DecodeStepConfig& c) : cfg_(c) {
     // serves batches of up to kFusedMaxBatch rows, and the shortest prompts where the multi-row
     // kernel takes them)
     const bool fused = cri::detail::prompt_attention_supported(cri::detail::kPromptAttnMinRows, c.head_dim);
-    const int64_t short_rows = std::min<int64_t>(MB, fused ? cri::detail::kPromptAttnMinRows - 1 : cri::detail::kPromptRows);
+    const int64_t short_rows =
+        std::min<int64_t>(MB, fused ? cri::detail::kPromptAttnMinRows - 1 : cri::detail::kPromptRows);
     prompt_mrow_ = fused && cri::detail::decode_attention_rows_mrow(kFusedMaxBatch + 1, c.head_dim);
     const int64_t arows = prompt_mrow_ ? short_rows : std::min<int64_t>(MB, kFusedMaxBatch);
     // the most records any batch size up to arows writes (its rows x heads x chunks; the chunk count

@@ -71,15 +71,22 @@ int cri_matmul(int format, const float* A, const void* B, float* C, int M, int N
  * above 16 rows the prefill GEMM's shapes with few output tiles (K % 256 == 0, e.g.
  * 512 x 2048 x 8192) -- store the partial sums in the workspace instead and add them in split
  * order in a second launch, so C has the same bits on every call (and the prefill shapes skip
- * the atomics and the zero fill: 512 x 2048 x 8192 Q4_K 41.1 -> 37.3 us).  Every other shape runs as
- * cri_matmul: 1..8 rows and unsplit products are deterministic there; above 16 rows with
- * K % 256 != 0 the k range may still be split with atomics.  workspace: device memory, 16-byte
- * aligned, at least cri_matmul_workspace_bytes(format, M, N, K) bytes; where it is used C must be
- * 16-byte aligned and N a multiple of 4 (CRI_ERR_ALIGNMENT otherwise).  Calls sharing a workspace
- * must be ordered on one stream. */
+ * the atomics and the zero fill: 512 x 2048 x 8192 Q4_K 41.1 -> 37.3 us).  Some prefill shapes that
+ * cri_matmul does not split (e.g. 2048 x 2048 x 8192 Q8_0) are faster split into a workspace on
+ * larger tiles (132 -> 108 us), and then are.  Every other shape runs as cri_matmul: 1..8 rows and
+ * unsplit products are deterministic there; above 16 rows with K % 256 != 0 the k range may still
+ * be split with atomics.
+ *
+ * workspace: device memory, 16-byte aligned, cri_matmul_workspace_bytes(format, M, N, K) bytes; C
+ * 16-byte aligned and N a multiple of 4.  For 2..16 rows and for the prefill shapes that cri_matmul
+ * splits this is required (CRI_ERR_INVALID_ARGUMENT for no workspace or one too small,
+ * CRI_ERR_ALIGNMENT).  For the prefill shapes that it does not split, a workspace that is missing,
+ * smaller or not so aligned is no error: the call runs as cri_matmul, whose sums are in another
+ * order.  So C's bits depend on the shape and on whether the advertised size and the alignment are
+ * given, and on nothing else.  Calls sharing a workspace must be ordered on one stream. */
 int cri_matmul_ws(int format, const float* A, const void* B, float* C, int M, int N, int K, void* workspace,
                   long long workspace_bytes, hipStream_t stream);
-/* bytes of workspace cri_matmul_ws uses for this shape (0 when it uses none; a negative
+/* the most bytes of workspace cri_matmul_ws uses for this shape (0 when it uses none; a negative
  * cri_status for invalid arguments) */
 long long cri_matmul_workspace_bytes(int format, int M, int N, int K);
 
@@ -156,13 +163,15 @@ int cri_fused_decode_attention_noalloc(const float* Q, const float* K_cache, con
                                        hipStream_t stream);
 /* Prompt attention over the [kv_len, n_kv_heads, head_dim] caches, the reference's prefill flow
  * (AttentionBlock::forward_from_qkv after the cache append, ref:src/attention.cu:809-871: Q K^T and
- * P V through batched_matmul_gqa around scale, causal mask and softmax): M query rows (already
+ * P V through batched_matmul_gqa around scale, causal mask and softmax), from 32 rows on at head_dim
+ * 64 and 128 as one kernel without materialized scores: M query rows (already
  * rotated) at Q + m * ldq, [n_heads * head_dim] each, at positions pos .. pos + M - 1; row m
  * attends to cache positions [0, pos + m]; output row m at output + m * n_heads * head_dim.  The
  * caches must hold rows 0 .. pos + M - 1 (rows past them are never read into the products).
  * head_dim a multiple of 4 up to 128, ldq a multiple of 4; K_cache, V_cache, output and the
  * workspace 16-byte aligned; workspace_bytes at least
- * cri_prefill_attention_workspace_bytes(M, n_heads, n_kv_heads, head_dim, pos + M). */
+ * cri_prefill_attention_workspace_bytes(M, n_heads, n_kv_heads, head_dim, pos + M), which is the size
+ * of the materialized flow's scores for every shape. */
 int cri_prefill_attention(const float* Q, int ldq, const float* K_cache, const float* V_cache, float* output, int M,
                           int n_heads, int n_kv_heads, int head_dim, int pos, float scale, void* workspace,
                           long long workspace_bytes, hipStream_t stream);

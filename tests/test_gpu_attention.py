@@ -260,10 +260,12 @@ def _oracle_rows(orc, q, kc, vc, H, Hkv, D, pos, scale):
 
 @pytest.mark.parametrize("H,Hkv,D,M,pos", [(32, 8, 64, 17, 0), (32, 8, 64, 64, 100), (32, 8, 64, 512, 0),
                                            (32, 8, 64, 512, 1400), (32, 8, 64, 600, 37), (4, 2, 128, 100, 30),
-                                           (8, 8, 32, 33, 5)])
+                                           (8, 8, 32, 33, 5), (8, 2, 96, 600, 37), (4, 1, 32, 513, 0)])
 def test_prefill_attention_matches_oracle(orc, H, Hkv, D, M, pos):
     # Q rows as the fused q/k/v projection leaves them (ldq = q + k + v widths); the cache rows past
-    # pos + M hold NaN, which no product may read; 600 rows run as two row blocks (512 + 88)
+    # pos + M hold NaN, which no product may read.  Head dims 64 and 128 run the prompt attention
+    # kernel from 32 rows on; the other shapes the products around a materialized softmax, 600 and 513
+    # rows of them as two row blocks (512 + 88, 512 + 1)
     rng = np.random.default_rng(M + pos + D)
     ldq = H * D + 2 * Hkv * D
     q = rng.standard_normal((M, ldq)).astype(np.float32)

@@ -399,9 +399,9 @@ def test_step_wide_models(orc, dim, M):
 
 @pytest.mark.parametrize("pos", [0, 1000])
 def test_prompt_two_layers_through_gqa(orc, pos):
-    # a 512-token prompt through two full-size Llama-3.2-1B layers: above 16 rows the step runs the
-    # reference's prefill flow (ref:src/attention.cu:809-871), Q K^T and P V on batched_matmul_gqa
-    # around a causal softmax (pinned on its own at 1e-5 in test_gpu_attention.py), with every
+    # a 512-token prompt through two full-size Llama-3.2-1B layers: the reference's prefill flow
+    # (ref:src/attention.cu:809-871) as the prompt attention kernel (pinned on its own at 1e-5 in
+    # test_gpu_attention.py and test_gpu_prompt_attention.py), with every
     # projection on the prefill GEMMs (fp16 operands; the stated bar 2e-3).  FP16 weights ~N(0, 0.02):
     # the random-block Q4_K weights of the other tests are not zero-mean (d sc q - dmin mn is mostly
     # positive), which gives q and k a large shared component, sharp attention rows, and a softmax
@@ -525,12 +525,12 @@ def test_batch_attention_rope_nan_cache(orc, M, pos):
     assert np.array_equal(b.cpu().numpy(), eager)
 
 
-@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("head_dim", [64, 128, 32])
 def test_prompt_row_blocks_nan_cache_and_replay(orc, head_dim):
-    # 600 rows: at head_dim 64 the multi-row split attention takes them at once, otherwise the
+    # 600 rows: at head_dim 64 and 128 the prompt attention kernel takes them at once, otherwise the
     # reference's flow on batched_matmul_gqa in two row blocks (512 + 88); cache rows past the
-    # step's positions hold NaN, which no product may read; a graph captured at one position (its
-    # products span the whole cache) and replayed at another equals the eager step there
+    # step's positions hold NaN, which no product may read; a graph captured at one position (the
+    # flow's products span the whole cache) and replayed at another equals the eager step there
     m = make_model(2, dim=512, n_heads=512 // head_dim, n_kv_heads=2, head_dim=head_dim, ffn=1024, vocab=900, seed=71,
                    fmts={n: "fp16" for n in ("q", "k", "v", "o", "gate", "up", "down")}, tok="q8_0", lm="fp16",
                    big_tables=False)
