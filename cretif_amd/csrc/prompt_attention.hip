@@ -44,7 +44,7 @@
 // A workgroup whose queries or tiles are not of that kind (kPaSpread), or lie near
 // the ends of fp32's range (a tile of K or V, or a query, holding an infinity, a
 // NaN or a value of 2^60, or whose largest magnitude is below 2^-50), takes fp32
-// products from the caches on v_mfma_f32_32x32x2_f32 instead (plain below).
+// products from the caches on v_mfma_f32_32x32x2_f32 instead (plain_group).
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -76,8 +76,8 @@ constexpr uint32_t kPaMax = 0x5D800000u, kPaMin = 0x26800000u;
 //     rows (and dims) a workgroup meets: then the large ones' share is off by 2^-27 of the small ones;
 //   * a value is off by 2^-38 of its tile's largest: 2^-28 of its own row's and dim's largest (a single value
 //     far below both is less exact than in fp32, by an amount that does not show in its row).
-// Measured with dims of K or V 2^8 apart, rows of V 2^8 apart, rows of K 2^6 apart or queries' dims 2^6 apart: 0.3 to
-// 0.75 of the fp32 products' error, in the 2-norm and in the largest error over the sum of an output's terms.
+// Measured with dims of K or V 2^8 apart, rows of V 2^8 apart, rows of K 2^6 apart or queries' dims 2^6 apart: 0.2 to
+// 0.8 of the fp32 products' error, in the 2-norm and in the largest error over the sum of an output's terms.
 // Rows and dims of zeros do not count, and dims only in tiles of at least kPaDimRows rows (with fewer, a
 // dim's largest is small by chance).
 constexpr int kPaSpread = 10;
@@ -153,9 +153,7 @@ __device__ __forceinline__ uint32_t halve_max(uint32_t a, uint32_t b, bool set) 
     return max(set ? b : a, dpp_bits<CTRL>(set ? a : b));
 }
 __device__ __forceinline__ int wave_max_int(int v) {
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) v = max(v, __shfl_xor(v, m));
-    return v;
+    return static_cast<int>(wave_max_bits(static_cast<uint32_t>(v) ^ 0x80000000u) ^ 0x80000000u);
 }
 // true when the parts of values with this largest magnitude are not good to 2^-24
 __device__ __forceinline__ bool out_of_range(uint32_t m) { return m >= kPaMax || (m != 0 && m < kPaMin); }
@@ -325,6 +323,78 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
     const RecPtr recs = (RecPtr)(a.recs + static_cast<long>(kvh) * a.ntiles);
     const int first_tile = t0 / kPaTile, last_tile = (Tmax - 1) / kPaTile;
 
+    // the waves of a query block meet in wave order: waves kw > 0 through LDS into wave 0, which writes the sums of
+    // the lanes' queries (row qm, head qg; o times back)
+    auto merge = [&](const float mx, const float l, paf16 (&o)[kDb], int qm, int qg, bool qok, float back) {
+        const float lq = l + shfl_xor32(l);
+        float* const mg = reinterpret_cast<float*>(lds);
+        float* const ml = mg + (KS - 1) * QB * 32 * pa_row(D);
+        __syncthreads();
+        if (kw > 0) {
+            const int slot = ((kw - 1) * QB + b) * 32 + i;
+            float* dst = mg + slot * pa_row(D) + 4 * h;
+#pragma unroll
+            for (int d = 0; d < kDb; ++d)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    *reinterpret_cast<f32x4*>(dst + 32 * d + 8 * v) =
+                        f32x4{o[d][4 * v], o[d][4 * v + 1], o[d][4 * v + 2], o[d][4 * v + 3]};
+            if (h == 0) {
+                ml[2 * slot] = mx;
+                ml[2 * slot + 1] = lq;
+            }
+        }
+        __syncthreads();
+        if (kw == 0 && qok) {
+            float M = mx;
+#pragma unroll
+            for (int x = 0; x < KS - 1; ++x) M = fmaxf(M, ml[2 * ((x * QB + b) * 32 + i)]);
+            float f = mx == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mx - M);
+            float L = f * lq;
+#pragma unroll
+            for (int d = 0; d < kDb; ++d) o[d] *= f;
+#pragma unroll
+            for (int x = 0; x < KS - 1; ++x) {
+                const int slot = (x * QB + b) * 32 + i;
+                const float mo = ml[2 * slot];
+                f = mo == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mo - M);
+                L = __builtin_fmaf(f, ml[2 * slot + 1], L);
+                const float* src = mg + slot * pa_row(D) + 4 * h;
+#pragma unroll
+                for (int d = 0; d < kDb; ++d)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const f32x4 y = *reinterpret_cast<const f32x4*>(src + 32 * d + 8 * v);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o[d][4 * v + e] = __builtin_fmaf(f, y[e], o[d][4 * v + e]);
+                    }
+            }
+            const int head = kvh * a.G + qg;
+            float* dst;
+            if (a.out) {
+                dst = a.out + qm * a.ldo + static_cast<long>(head) * D + 4 * h;
+            } else {
+                float* r = a.part + ((static_cast<long>(qm) * a.G * a.n_kv + head) * a.nchunks + c) * (D + 4);
+                if (h == 0) {
+                    r[0] = M;
+                    r[1] = L;
+                }
+                dst = r + 4 + 4 * h;
+            }
+            const float den = a.out ? L : 1.0f;
+#pragma unroll
+            for (int d = 0; d < kDb; ++d)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    f32x4 y;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) y[e] = o[d][4 * v + e] / den * back;
+                    *reinterpret_cast<f32x4*>(dst + 32 * d + 8 * v) = y;
+                }
+        }
+    };
+
+    // one query group; false (and nothing written) where its operands are not for the parts
     auto run_group = [&](const int grp) {
         const int q0 = grp * 32 * QB + 32 * b;  // the wave's queries q0 .. q0 + 31
         const int q = q0 + i;
@@ -355,7 +425,7 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
             for (int ks = 0; ks < kKs; ++ks)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) qmx = max(qmx, absbits(x[ks][e]));
-            qmx = max(qmx, static_cast<uint32_t>(__shfl_xor(static_cast<int>(qmx), 32)));
+            qmx = max32(qmx);
             const int qe = out_of_range(qmx) ? 0 : scale_exp(qmx);
             qinv = pow2(-qe);
 #pragma unroll
@@ -369,26 +439,27 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
         // the records of every tile the workgroup sees: a flag, or magnitudes too far apart, or scores too
         // large, or queries out of range take the fp32 path; E is the scale of the accumulators
         int E;
-        bool slow = out_of_range(qmx);
         {
-            float kfm = 0.0f;  // of the largest |k|
+            bool slow = out_of_range(qmx);
+            uint32_t kfm = 0;  // bits of the factor of the largest |k|
             int lo = -(1 << 20), hi = -(1 << 20);  // -(least exponent), largest exponent
             const PaTile* r = a.recs + static_cast<long>(kvh) * a.ntiles;
             for (int t = first_tile + lane; t * kPaTile < end; t += 64) {
                 slow |= r[t].bad != 0;
-                kfm = fmaxf(kfm, r[t].kf);
+                kfm = max(kfm, absbits(r[t].kf));
                 if (r[t].ve != kPaNoScale) {
                     lo = max(lo, -r[t].ve);
                     hi = max(hi, r[t].vs);
                 }
             }
-            kfm = wave_max(kfm);
-            slow |= qinv * kfm > pow2(kPaScore - 28);  // the magnitudes are below 2^14 times qinv and kfm
+            kfm = wave_max_bits(kfm);
+            // the magnitudes are below 2^14 times qinv and kfm
+            slow |= qinv * __builtin_bit_cast(float, kfm) > pow2(kPaScore - 28);
             lo = -wave_max_int(lo);
             hi = wave_max_int(hi);
             E = __builtin_amdgcn_readfirstlane(lo == 1 << 20 ? 0 : lo);
             slow |= hi - lo > kPaSpread;
-            slow = __syncthreads_or(slow);  // (also: the previous group's merge has been read)
+            if (__syncthreads_or(slow)) return false;  // (also: the previous group's merge has been read)
         }
 
         // the K or V half of stage st's tiles into buffer st & 1; the waves share the copies
@@ -494,114 +565,6 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
         };
         const char* const mine = lds + kw * kHalf + 16 * lane;
         int tb = t0 + kw * kPaTile;
-        // The same tiles with fp32 products, in the same transposed layout: the n-th instruction of S^T takes dim
-        // 8 (n >> 2) + 4 h + (n & 3) from lane (i, h) for key i and query i, the n-th of a dim block of O^T position
-        // 8 (n >> 2) + 4 h + (n & 3), whose probability the lane holds in its n-th score.  Bound by the matrix
-        // instructions and, its loads hidden by the SIMD's other wave only, their latency: every query of 2048 rows,
-        // 32/8 heads of 64, 249 us (the five launches over materialized scores 591, one query at a time on scalar
-        // FMAs 18300); heads of 128 481 (768, 33500); 64 rows 17 (32, 262).
-        auto plain = [&]() {
-            const long row = static_cast<long>(a.n_kv) * D;
-            const float *const Kh = a.K + kvh * D + 4 * h, *const Vh = a.V + kvh * D;
-            const float* const qp = a.Q + qm * a.ldq + static_cast<long>(kvh * a.G + qg) * D + 4 * h;
-            float* const ps = reinterpret_cast<float*>(lds) + w * 2048;  // [32 positions][32 queries], then [..][dims]
-            static_assert(pa_lds_bytes<D, QB, KS>() >= kWaves * 8192);
-            const int hi = q0 < nq ? min(Tb + min(q0 + 31, nq - 1) / a.G, t1) : t0;  // the wave's last limit
-            for (; tb < hi; tb += kStagePos) {
-                const float* const kp = Kh + min(tb + i, Tmax - 1) * row;
-                paf16 sa, sb;  // two chains
-#pragma unroll
-                for (int v = 0; v < 16; ++v) sa[v] = sb[v] = 0.0f;
-#pragma unroll
-                for (int c = 0; c < D / 64; ++c) {
-                    // (the query is read again for every tile: at head_dim 128 there is no room to keep it)
-                    if constexpr (D > 64) asm volatile("" ::: "memory");
-                    f32x4 k[8], qv[8];
-#pragma unroll
-                    for (int n = 0; n < 8; ++n) k[n] = ld_f32x4(kp + 64 * c + 8 * n);
-#pragma unroll
-                    for (int n = 0; n < 8; ++n) qv[n] = ld_f32x4(qp + 64 * c + 8 * n);
-#pragma unroll
-                    for (int n = 0; n < 8; ++n) {
-                        sa = __builtin_amdgcn_mfma_f32_32x32x2f32(k[n].x, qv[n].x, sa, 0, 0, 0);
-                        sb = __builtin_amdgcn_mfma_f32_32x32x2f32(k[n].y, qv[n].y, sb, 0, 0, 0);
-                        sa = __builtin_amdgcn_mfma_f32_32x32x2f32(k[n].z, qv[n].z, sa, 0, 0, 0);
-                        sb = __builtin_amdgcn_mfma_f32_32x32x2f32(k[n].w, qv[n].w, sb, 0, 0, 0);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                float p[16], tmax = -INFINITY;
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    p[v] = tb + 8 * (v >> 2) + 4 * h + (v & 3) < lim ? (sa[v] + sb[v]) * a.qscale : -INFINITY;
-                    tmax = fmaxf(tmax, p[v]);
-                }
-                const float mnew = fmaxf(mx, fmaxf(tmax, shfl_xor32(tmax)));
-                const float base = mnew == -INFINITY ? 0.0f : mnew;
-                const float cf = __builtin_amdgcn_exp2f(mx - base);
-                mx = mnew;
-                l *= cf;
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    p[v] = __builtin_amdgcn_exp2f(p[v] - base);
-                    l += p[v];
-                }
-#pragma unroll
-                for (int d = 0; d < kDb; ++d) o[d] *= cf;
-#pragma unroll
-                for (int d0 = 0; d0 < kDb; d0 += 2) {
-                    float x[2][16];
-                    bool odd = false;
-#pragma unroll
-                    for (int n = 0; n < 16; ++n) {
-                        const float* const vp =
-                            Vh + min(tb + 8 * (n >> 2) + 4 * h + (n & 3), Tmax - 1) * row + 32 * d0 + i;
-#pragma unroll
-                        for (int d = 0; d < 2; ++d) {
-                            x[d][n] = vp[32 * d];
-                            odd |= absbits(x[d][n]) >= 0x7F800000u;
-                        }
-                    }
-                    if (tb + kPaTile > lim_lo && __any(odd)) {
-                        // an infinite or NaN value that not every query sees: times the probability 0 of those
-                        // that do not, it would reach them
-#pragma unroll
-                        for (int d = 0; d < 2; ++d) {
-#pragma unroll
-                            for (int v = 0; v < 16; ++v) {
-                                ps[32 * (8 * (v >> 2) + 4 * h + (v & 3)) + i] = p[v];
-                                ps[32 * (32 + 8 * (v >> 2) + 4 * h + (v & 3)) + i] = x[d][v];
-                            }
-                            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                            __builtin_amdgcn_wave_barrier();
-#pragma unroll 4
-                            for (int u = 0; u < kPaTile; ++u) {
-                                const float pu = ps[32 * u + i];
-                                const uint32_t seen = tb + u < lim ? ~0u : 0u;  // (a select would become branches)
-#pragma unroll
-                                for (int v = 0; v < 4; ++v) {
-                                    const u32x4 y =
-                                        *reinterpret_cast<const u32x4*>(ps + 32 * (32 + u) + 8 * v + 4 * h) & seen;
-                                    const f32x4 z = __builtin_bit_cast(f32x4, y);
-#pragma unroll
-                                    for (int e = 0; e < 4; ++e)
-                                        o[d0 + d][4 * v + e] = __builtin_fmaf(pu, z[e], o[d0 + d][4 * v + e]);
-                                }
-                            }
-                            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                            __builtin_amdgcn_wave_barrier();
-                        }
-                    } else {
-#pragma unroll
-                        for (int n = 0; n < 16; ++n)
-#pragma unroll
-                            for (int d = 0; d < 2; ++d)
-                                o[d0 + d] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[d][n], p[n], o[d0 + d], 0, 0, 0);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-        };
         // stage st (position J = st & 1 of the buffers); r: its tile's record, the next one's when it returns
         auto stage = [&](int st, auto pos, float& kf, int& ve, paf16& s, paf16& sn) {
             constexpr int J = decltype(pos)::value;
@@ -621,9 +584,7 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
             ve = ven;
             tb += kStagePos;
         };
-        if (slow) {
-            plain();
-        } else if (nst > 0) {
+        if (nst > 0) {
             paf16 s0, s1;
             float kf = recs[rec_of(0)].kf;
             int ve = recs[rec_of(0)].ve;
@@ -640,78 +601,141 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
             }
         }
 
-        // the waves of a query block meet in wave order: waves kw > 0 through LDS into wave 0
-        const float lq = l + shfl_xor32(l);
-        float* const mg = reinterpret_cast<float*>(lds);
-        float* const ml = mg + (KS - 1) * QB * 32 * pa_row(D);
-        __syncthreads();
-        if (kw > 0) {
-            const int slot = ((kw - 1) * QB + b) * 32 + i;
-            float* dst = mg + slot * pa_row(D) + 4 * h;
-#pragma unroll
-            for (int d = 0; d < kDb; ++d)
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    *reinterpret_cast<f32x4*>(dst + 32 * d + 8 * v) =
-                        f32x4{o[d][4 * v], o[d][4 * v + 1], o[d][4 * v + 2], o[d][4 * v + 3]};
-            if (h == 0) {
-                ml[2 * slot] = mx;
-                ml[2 * slot + 1] = lq;
-            }
-        }
-        __syncthreads();
-        if (kw == 0 && qok) {
-            float M = mx;
-#pragma unroll
-            for (int x = 0; x < KS - 1; ++x) M = fmaxf(M, ml[2 * ((x * QB + b) * 32 + i)]);
-            float f = mx == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mx - M);
-            float L = f * lq;
-#pragma unroll
-            for (int d = 0; d < kDb; ++d) o[d] *= f;
-#pragma unroll
-            for (int x = 0; x < KS - 1; ++x) {
-                const int slot = (x * QB + b) * 32 + i;
-                const float mo = ml[2 * slot];
-                f = mo == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mo - M);
-                L = __builtin_fmaf(f, ml[2 * slot + 1], L);
-                const float* src = mg + slot * pa_row(D) + 4 * h;
-#pragma unroll
-                for (int d = 0; d < kDb; ++d)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const f32x4 y = *reinterpret_cast<const f32x4*>(src + 32 * d + 8 * v);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) o[d][4 * v + e] = __builtin_fmaf(f, y[e], o[d][4 * v + e]);
-                    }
-            }
-            // the accumulators hold 2^(kShift + E) times the sums, or the sums
-            const float back = slow ? 1.0f : pow2(-E - kShift);
-            const int head = kvh * a.G + qg;
-            float* dst;
-            if (a.out) {
-                dst = a.out + qm * a.ldo + static_cast<long>(head) * D + 4 * h;
-            } else {
-                float* r = a.part + ((static_cast<long>(qm) * a.G * a.n_kv + head) * a.nchunks + c) * (D + 4);
-                if (h == 0) {
-                    r[0] = M;
-                    r[1] = L;
-                }
-                dst = r + 4 + 4 * h;
-            }
-            const float den = a.out ? L : 1.0f;
-#pragma unroll
-            for (int d = 0; d < kDb; ++d)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    f32x4 y;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) y[e] = o[d][4 * v + e] / den * back;
-                    *reinterpret_cast<f32x4*>(dst + 32 * d + 8 * v) = y;
-                }
-        }
+        merge(mx, l, o, qm, qg, qok, pow2(-E - kShift));
+        return true;
     };
-    run_group(grp0);
-    if (a.paired && ngrp - 1 - grp0 != grp0) run_group(ngrp - 1 - grp0);
+    // The same group with fp32 products, in the same transposed layout: the n-th instruction of S^T takes dim
+    // 8 (n >> 2) + 4 h + (n & 3) from lane (i, h) for key i and query i, the n-th of a dim block of O^T position
+    // 8 (n >> 2) + 4 h + (n & 3), whose probability the lane holds in its n-th score.  Bound by the matrix
+    // instructions and, its loads hidden by the SIMD's other wave only, their latency: every query of 2048 rows,
+    // 32/8 heads of 64, 250 us (the five launches over materialized scores 591, one query at a time on scalar
+    // FMAs 18300); heads of 128 490 (768, 33500); 64 rows 17 (32, 262).
+    auto plain_group = [&](const int grp) {
+        const int q0 = grp * 32 * QB + 32 * b, q = q0 + i;
+        const bool qok = q < nq;
+        const int qm = qok ? q / a.G : 0, qg = qok ? q - qm * a.G : 0;
+        const int lim = qok ? min(Tb + qm, t1) : t1, lim_lo = min(Tb + min(q0, nq - 1) / a.G, t1);
+        float mx = -INFINITY, l = 0.0f;
+        paf16 o[kDb];
+#pragma unroll
+        for (int d = 0; d < kDb; ++d)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) o[d][v] = 0.0f;
+        const long row = static_cast<long>(a.n_kv) * D;
+        const float *const Kh = a.K + kvh * D + 4 * h, *const Vh = a.V + kvh * D;
+        const float* const qp = a.Q + qm * a.ldq + static_cast<long>(kvh * a.G + qg) * D + 4 * h;
+        float* const ps = reinterpret_cast<float*>(lds) + w * 2048;  // [32 positions][32 queries], then [..][dims]
+        static_assert(pa_lds_bytes<D, QB, KS>() >= kWaves * 8192);
+        const int hi = q0 < nq ? min(Tb + min(q0 + 31, nq - 1) / a.G, t1) : t0;  // the wave's last limit
+        for (int tb = t0 + kw * kPaTile; tb < hi; tb += kStagePos) {
+            const float* const kp = Kh + min(tb + i, Tmax - 1) * row;
+            paf16 sa, sb;  // two chains
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sa[v] = sb[v] = 0.0f;
+#pragma unroll
+            for (int c = 0; c < D / 64; ++c) {
+                // (the query is read again for every tile: at head_dim 128 there is no room to keep it)
+                if constexpr (D > 64) asm volatile("" ::: "memory");
+                f32x4 k[8], qv[8];
+#pragma unroll
+                for (int n = 0; n < 8; ++n) k[n] = ld_f32x4(kp + 64 * c + 8 * n);
+#pragma unroll
+                for (int n = 0; n < 8; ++n) qv[n] = ld_f32x4(qp + 64 * c + 8 * n);
+#pragma unroll
+                for (int n = 0; n < 8; ++n) {
+                    sa = __builtin_amdgcn_mfma_f32_32x32x2f32(k[n].x, qv[n].x, sa, 0, 0, 0);
+                    sb = __builtin_amdgcn_mfma_f32_32x32x2f32(k[n].y, qv[n].y, sb, 0, 0, 0);
+                    sa = __builtin_amdgcn_mfma_f32_32x32x2f32(k[n].z, qv[n].z, sa, 0, 0, 0);
+                    sb = __builtin_amdgcn_mfma_f32_32x32x2f32(k[n].w, qv[n].w, sb, 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            float p[16], tmax = -INFINITY;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                p[v] = tb + 8 * (v >> 2) + 4 * h + (v & 3) < lim ? (sa[v] + sb[v]) * a.qscale : -INFINITY;
+                tmax = fmaxf(tmax, p[v]);
+            }
+            const float mnew = fmaxf(mx, fmaxf(tmax, shfl_xor32(tmax)));
+            const float base = mnew == -INFINITY ? 0.0f : mnew;
+            const float cf = __builtin_amdgcn_exp2f(mx - base);
+            mx = mnew;
+            l *= cf;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                p[v] = __builtin_amdgcn_exp2f(p[v] - base);
+                l += p[v];
+            }
+#pragma unroll
+            for (int d = 0; d < kDb; ++d) o[d] *= cf;
+#pragma unroll
+            for (int d0 = 0; d0 < kDb; d0 += 2) {
+                float x[2][16];
+                bool odd = false;
+#pragma unroll
+                for (int n = 0; n < 16; ++n) {
+                    const float* const vp =
+                        Vh + min(tb + 8 * (n >> 2) + 4 * h + (n & 3), Tmax - 1) * row + 32 * d0 + i;
+#pragma unroll
+                    for (int d = 0; d < 2; ++d) {
+                        x[d][n] = vp[32 * d];
+                        odd |= absbits(x[d][n]) >= 0x7F800000u;
+                    }
+                }
+                if (tb + kPaTile > lim_lo && __any(odd)) {
+                    // an infinite or NaN value that not every query sees: times the probability 0 of those
+                    // that do not, it would reach them
+#pragma unroll
+                    for (int d = 0; d < 2; ++d) {
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) {
+                            ps[32 * (8 * (v >> 2) + 4 * h + (v & 3)) + i] = p[v];
+                            ps[32 * (32 + 8 * (v >> 2) + 4 * h + (v & 3)) + i] = x[d][v];
+                        }
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+#pragma unroll 4
+                        for (int u = 0; u < kPaTile; ++u) {
+                            const float pu = ps[32 * u + i];
+                            const uint32_t seen = tb + u < lim ? ~0u : 0u;  // (a select would become branches)
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) {
+                                const u32x4 y =
+                                    *reinterpret_cast<const u32x4*>(ps + 32 * (32 + u) + 8 * v + 4 * h) & seen;
+                                const f32x4 z = __builtin_bit_cast(f32x4, y);
+#pragma unroll
+                                for (int e = 0; e < 4; ++e)
+                                    o[d0 + d][4 * v + e] = __builtin_fmaf(pu, z[e], o[d0 + d][4 * v + e]);
+                            }
+                        }
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                    }
+                } else {
+#pragma unroll
+                    for (int n = 0; n < 16; ++n)
+#pragma unroll
+                        for (int d = 0; d < 2; ++d)
+                            o[d0 + d] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[d][n], p[n], o[d0 + d], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        merge(mx, l, o, qm, qg, qok, 1.0f);
+    };
+    const int grp1 = a.paired ? ngrp - 1 - grp0 : grp0;
+    const bool ok0 = run_group(grp0), ok1 = grp1 == grp0 ? ok0 : run_group(grp1);
+    if (ok0 && ok1) return;
+    // (apart from the groups above and once for both: inside them it cost every call of head_dim 128 1 us, with one
+    // loop around everything 5)
+    int grp = ok0 ? grp1 : grp0;
+#pragma clang loop unroll(disable)
+    while (true) {
+        __syncthreads();  // a merge before has been read
+        plain_group(grp);
+        if (grp == grp1 || ok1) break;
+        grp = grp1;
+    }
 }
 
 }  // namespace
