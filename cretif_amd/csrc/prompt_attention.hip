@@ -725,7 +725,7 @@ __global__ __launch_bounds__(64 * QB * KS) __attribute__((amdgpu_waves_per_eu(2,
     };
     const int grp1 = a.paired ? ngrp - 1 - grp0 : grp0;
     const bool ok0 = run_group(grp0), ok1 = grp1 == grp0 ? ok0 : run_group(grp1);
-    if (ok0 && ok1) return;
+    if (__builtin_expect(ok0 && ok1, 1)) return;
     // (apart from the groups above and once for both: inside them it cost every call of head_dim 128 1 us, with one
     // loop around everything 5)
     int grp = ok0 ? grp1 : grp0;
